@@ -122,7 +122,7 @@ Kernels pick_kernel(const SimplerHipPaDecodeArgs *a, bool append = false) {
         if (append) s.ka = f16 ? pick_gqa_f16_append(bs, dk, out) : pick_gqa_bf16_append(bs, dk, out);
     }
     s.merge = pick_merge(dv, out);
-    if (!s.merge.fn || (append && !s.ka.main)) s.k.main = nullptr;
+    if (!s.merge.fn[0] || (append && !s.ka.main)) s.k.main = nullptr;
     return s;
 }
 
@@ -268,6 +268,42 @@ Plan make_plan(const SimplerHipPaDecodeArgs *a, const KernelPair &k) {  // k: th
     return p;
 }
 
+// The merge's launch: workgroups per tile (grid y), each with `units` of the
+// tile's 16-byte units. A tile is cut into about workers / tiles + 1 pieces.
+// It is shared out among workgroups (down to 8 units, a 128-byte line, each)
+// until a thread has one unit and reads kMergeAhead of its pieces at most,
+// as long as the grid stays within kMergeGrid workgroups: with more, every
+// workgroup's own set-up costs more than its shorter chain saves (128 x 128
+// MLA heads, 1024 tiles: 24.1 us with four per tile, 14.6 with one; 256
+// tiles: 14.6 against 19.9; one sequence of 16 heads and 32000 tokens, one
+// tile: 8 us in 128 workgroups, 321 in one). Small tiles of few pieces take
+// smaller workgroups.
+struct MergePlan {
+    KernelFn fn;
+    int units, groups, threads;
+};
+constexpr int64_t kMergeGrid = 1024;
+
+MergePlan plan_merge(const MergeFn &m, const SimplerHipPaDecodeArgs *a, const Plan &p) {
+    const int64_t all = (int64_t)std::min(16, p.rows) * (a->head_dim_v / 4);
+    const int64_t lists = (int64_t)a->batch * a->num_kv_heads;
+    const int64_t tiles = std::max<int64_t>(lists * p.row_tiles, 1);
+    const int64_t pieces = p.workers / std::max<int64_t>(lists * p.row_groups, 1) + 1;
+    MergePlan r{};
+    int64_t units = all, groups = 1;
+    while (units >= 16 && tiles * groups * 2 <= kMergeGrid &&
+           (units > kMergeThreads || units * pieces > kMergeThreads * kMergeAhead)) {
+        units = (units + 1) / 2;
+        groups = (all + units - 1) / units;
+    }
+    r.units = (int)units;
+    r.groups = (int)groups;
+    r.threads = kMergeThreads;
+    while (r.threads > 128 && units <= r.threads / 2 && units * pieces <= r.threads / 2 * kMergeAhead) r.threads /= 2;
+    r.fn = m.fn[units <= kMergeThreads ? 0 : units <= 2 * kMergeThreads ? 1 : 2];
+    return r;
+}
+
 }  // namespace
 }  // namespace simpler_hip
 
@@ -390,14 +426,16 @@ int pa_decode_launch(const SimplerHipPaDecodeArgs *a, void *workspace, size_t wo
     P.v_new = (const uint16_t *)v_new;
 
     const int64_t tiles = (int64_t)a->batch * a->num_kv_heads * plan.row_tiles;
+    const MergePlan merge = plan_merge(s.merge, a, plan);
+    P.merge_units = merge.units;
     if (phases & SIMPLER_HIP_PHASE_MAIN) {
         hipLaunchKernelGGL(plan.main, dim3((unsigned)plan.grid), dim3((unsigned)plan.threads), (unsigned)plan.lds,
                            (hipStream_t)stream, P);
         if (hipGetLastError() != hipSuccess) return SIMPLER_HIP_ERR_LAUNCH;
     }
     if (phases & SIMPLER_HIP_PHASE_MERGE) {
-        hipLaunchKernelGGL(s.merge.fn, dim3((unsigned)tiles), dim3((unsigned)s.merge.threads), 0, (hipStream_t)stream,
-                           P);
+        hipLaunchKernelGGL(merge.fn, dim3((unsigned)tiles, (unsigned)merge.groups), dim3((unsigned)merge.threads), 0,
+                           (hipStream_t)stream, P);
         if (hipGetLastError() != hipSuccess) return SIMPLER_HIP_ERR_LAUNCH;
     }
     return SIMPLER_HIP_OK;

@@ -130,6 +130,7 @@ struct KernelParams {
     // null for MLA (V is a prefix of K). Null when not appending.
     const uint16_t *k_new;
     const uint16_t *v_new;
+    int32_t merge_units;  // merge kernel: 16-byte units of a tile per workgroup
 };
 
 __device__ __forceinline__ u32x4_t ld16(const uint16_t *p) { return *reinterpret_cast<const u32x4_t *>(p); }
@@ -1520,26 +1521,46 @@ __global__ void __launch_bounds__(64 * MAXW) pa_decode_kernel(const KernelParams
 // (pa_kernel.cce:1666-1773 CombineScale), and zeros for empty contexts.
 // ---------------------------------------------------------------------------
 
-// Threads per merge workgroup: one 16-byte unit of a tile's 16 x DV output per
-// thread up to DV = 128 (512 threads), four per thread for MLA's DV = 512.
-template <int DV> constexpr int merge_threads() { return DV * 4 < 512 ? (DV * 4 < 64 ? 64 : DV * 4) : 512; }
-constexpr int kMergeLdsPieces = 32;  // pieces per tile merged through LDS weights
+constexpr int kMergeThreads = 512;  // largest merge workgroup
+constexpr int kMergeAhead = 8;     // 16-byte units a thread reads before the weights are known
+constexpr int kMergeTable = 2048;  // (row, piece) weights a workgroup holds in LDS
 
-template <int DV, typename OutT>
-// MLA (DV = 512): every tile of a launch is cut, and 1024 of them (cfg4) fit
-// the chip at once only at eight waves per SIMD, i.e. 64 registers, hence one
-// piece read ahead (measured 24.9 -> 23.2 us against four waves per SIMD with
-// four read ahead).
-__global__ void __launch_bounds__(merge_threads<DV>()) __attribute__((amdgpu_waves_per_eu(DV >= 512 ? 8 : 1)))
+// Combines x over a row of 16 lanes (DPP rotations); every lane gets the result.
+template <typename F>
+__device__ __forceinline__ float row16_combine(float x, F f) {
+#define SIMPLER_ROR(n) \
+    f(x, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x120 + n, 0xf, 0xf, false)))
+    x = SIMPLER_ROR(8);
+    x = SIMPLER_ROR(4);
+    x = SIMPLER_ROR(2);
+    x = SIMPLER_ROR(1);
+#undef SIMPLER_ROR
+    return x;
+}
+
+// O = sum_w e^{m_w - M} O_w / L over a tile's pieces w. The merge is bound by
+// memory latency (kernel arguments, lengths, pieces: three round trips), so
+// every piece load that can be is in flight at once. A tile's 16-byte units
+// (rows x DV / 4) are shared out over the grid's y workgroups, merge_units
+// each (the host sizes it so that a thread's share of pieces fits
+// kMergeAhead loads). A thread owns UPT units; a workgroup with fewer units
+// than threads and more than kMergeAhead pieces runs groups of threads over
+// the same units, group g taking every G-th piece, whose sums meet in LDS.
+// The weights are worked out in LDS while the pieces are in flight.
+// One workgroup per tile whatever its pieces, as before, left a long context
+// of few sequences to a few CUs: 32 sequences of 16 MLA heads 20 -> 7.6 us.
+template <int DV, typename OutT, int UPT>
+__global__ void __launch_bounds__(kMergeThreads) __attribute__((amdgpu_waves_per_eu(UPT == 4 ? 8 : 4)))
 pa_merge_kernel(const KernelParams P) {
-    constexpr int MT = merge_threads<DV>();
-    constexpr int UNITS = 16 * (DV / 4);        // 16-byte units of a full tile
-    constexpr int UPT = (UNITS + MT - 1) / MT;  // units per thread
-    constexpr int PRE = UPT == 1 ? 8 : (DV >= 512 ? 1 : 4);  // pieces per unit read before the weights are known
-    const int tid = threadIdx.x;
+    constexpr int UPR = DV / 4;  // units per row
+    // Pieces of each unit read ahead. With four units per thread the shape is
+    // MLA's, thousands of workgroups of two or three pieces each: eight waves
+    // per SIMD (64 registers) and one piece ahead.
+    constexpr int PRE = UPT == 4 ? 1 : kMergeAhead / UPT;
+    const int tid = threadIdx.x, MT = blockDim.x;
     // The main kernel is done: hand its error word to the host through
     // pinned memory (a run's wait then needs no device-to-host copy).
-    if (P.err_mirror && blockIdx.x == 0 && tid == 0)
+    if (P.err_mirror && blockIdx.x == 0 && blockIdx.y == 0 && tid == 0)
         __hip_atomic_store(P.err_mirror, __hip_atomic_load(P.error_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT),
                            __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     const int tpb = P.kv_heads * P.row_tiles;
@@ -1550,16 +1571,20 @@ pa_merge_kernel(const KernelParams P) {
     const int jt = kvh * P.row_groups + rg;  // tile of the batch in the work lists
     const int list = list_of_tile(P, jt / lane_tiles(P), b), j = jt - (jt / lane_tiles(P)) * lane_tiles(P);
     const int rows_here = min(16, P.rows - rt * 16);
+    const int unit0 = blockIdx.y * P.merge_units;
+    const int units = min(P.merge_units, rows_here * UPR - unit0);  // of this workgroup
+    if (units <= 0) return;  // a last tile with fewer rows
     int prefix = 0;
     int ctxb = 0;
     const int total = scan_work(P, b, &prefix, &ctxb, -1, nullptr, nullptr, nullptr);
     const int nb = (ctxb + P.block_size - 1) / P.block_size;
+    auto out_at = [&](int unit) {  // its output element
+        const int row = unit / UPR;
+        return out_row_offset(P, b, kvh, rt * 16 + row, DV) + 4 * (unit - row * UPR);
+    };
     if (nb == 0) {  // empty context: defined as a zero output
-        for (int idx = tid; idx < rows_here * (DV / 4); idx += MT) {
-            const int row = idx / (DV / 4), c4 = idx - row * (DV / 4);
-            OutStore<OutT>::store4(P.out, out_row_offset(P, b, kvh, rt * 16 + row, DV) + 4 * c4,
-                                   (f32x4_t){0.f, 0.f, 0.f, 0.f});
-        }
+        for (int u = tid; u < units; u += MT)
+            OutStore<OutT>::store4(P.out, out_at(unit0 + u), (f32x4_t){0.f, 0.f, 0.f, 0.f});
         return;
     }
     const int per_list = max(P.workers / P.lanes, 1);
@@ -1568,89 +1593,108 @@ pa_merge_kernel(const KernelParams P) {
     const int tb = t0 + P.seg_cost;                 // its first block's
     const int w_first = tb / chunk, w_last = (tb + nb - 1) / chunk;  // slices of the list
     if (w_first == w_last) return;  // a tile inside one slice is finished by the main kernel
-    // Log-sum-exp over the pieces: the row max and total l from the (m, l)
-    // pairs first, then O = sum_w e^{m_w - M} O_w / L, whose piece loads do not
-    // depend on each other and stay in flight together.
-    auto piece_of = [&](int c) -> int64_t {
-        const int slot = (c * chunk >= t0) ? 0 : 1;
-        const int64_t w = (int64_t)c * P.lanes + list;  // the worker that ran slice c
-        return (w * P.tiles_per_worker + wave) * 2 + slot;
-    };
     const int np = w_last - w_first + 1;
-    if (np <= kMergeLdsPieces) {
-        // Per-(row, piece) weights e^{m_w - M} / L once per workgroup, then the
-        // partial rows stream through with no dependent loads in the way. Every
-        // unit of the thread has its first PRE pieces read together with the
-        // (m, l) loads: they do not depend on the weights, so the merge is one
-        // memory round trip after the work scan, not one per unit.
-        __shared__ float wgt[16][kMergeLdsPieces];  // m of each (row, piece), then its weight
-        __shared__ float lsum[16][kMergeLdsPieces];
-        const int units = rows_here * (DV / 4);
-        f32x4_t pre[UPT][PRE];
-#pragma unroll
-        for (int u = 0; u < UPT; ++u) {
-            const int idx = tid + u * MT;
-            const int row = idx / (DV / 4), c4 = idx - row * (DV / 4);
-#pragma unroll
-            for (int k = 0; k < PRE; ++k)
-                pre[u][k] = (idx < units && k < np)
-                                ? *reinterpret_cast<const f32x4_t *>(P.part_o + (piece_of(w_first + k) * 16 + row) * DV +
-                                                                     4 * c4)
-                                : (f32x4_t){0.f, 0.f, 0.f, 0.f};
-        }
-        for (int e = tid; e < 16 * np; e += MT) {  // all (m, l) loads in flight at once
-            const int row = e / np, k = e - row * np;
-            const int64_t pc = piece_of(w_first + k);
-            wgt[row][k] = P.part_ml[pc * 32 + row];
-            lsum[row][k] = P.part_ml[pc * 32 + 16 + row];
-        }
-        __syncthreads();
-        if (tid < 16) {
+    // Piece k is the part of the tile run by slice w_first + k of the list,
+    // the worker (w_first + k) * lanes + list: slot 1 of the first one if its
+    // slice began before the tile, else slot 0. Pieces are a fixed number of
+    // slots apart.
+    const int64_t first = (((int64_t)w_first * P.lanes + list) * P.tiles_per_worker + wave) * 2;
+    const int64_t step = (int64_t)P.lanes * P.tiles_per_worker * 2;
+    const int slot0 = w_first * chunk >= t0 ? 0 : 1;
+    const float *const o_base = P.part_o + first * 16 * DV, *const ml_base = P.part_ml + first * 32;
+    auto piece_unit = [&](int k, int unit) -> f32x4_t {
+        return *reinterpret_cast<const f32x4_t *>(o_base + (k * step + (k == 0 ? slot0 : 0)) * (16 * DV) + 4 * unit);
+    };
+    auto piece_ml = [&](int k, int row) { return ml_base + (k * step + (k == 0 ? slot0 : 0)) * 32 + row; };
+
+    const int r0 = unit0 / UPR, nr = (unit0 + units - 1) / UPR - r0 + 1;  // its rows
+    if (nr * np > kMergeTable) {  // contexts cut finer than the default plans cut
+        for (int u = tid; u < units; u += MT) {
+            const int row = (unit0 + u) / UPR;
             float M = -INFINITY;
-            for (int k = 0; k < np; ++k) M = fmaxf(M, wgt[tid][k]);
+            for (int k = 0; k < np; ++k) M = fmaxf(M, *piece_ml(k, row));
             float L = 0.f;
-            for (int k = 0; k < np; ++k) {
-                const float c = __expf(wgt[tid][k] - M);
-                wgt[tid][k] = c;
-                L += c * lsum[tid][k];
-            }
-            const float inv = L > 0.f ? 1.f / L : 0.f;
-            for (int k = 0; k < np; ++k) wgt[tid][k] *= inv;
-        }
-        __syncthreads();
-#pragma unroll
-        for (int u = 0; u < UPT; ++u) {
-            const int idx = tid + u * MT;
-            if (idx >= units) break;
-            const int row = idx / (DV / 4), c4 = idx - row * (DV / 4);
             f32x4_t o = (f32x4_t){0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int k = 0; k < PRE; ++k)
-                if (k < np) o += wgt[row][k] * pre[u][k];
 #pragma unroll 4
-            for (int k = PRE; k < np; ++k) {
-                const int64_t piece = piece_of(w_first + k);
-                o += wgt[row][k] * *reinterpret_cast<const f32x4_t *>(P.part_o + (piece * 16 + row) * DV + 4 * c4);
+            for (int k = 0; k < np; ++k) {
+                const float c = __expf(*piece_ml(k, row) - M);
+                L += c * piece_ml(k, row)[16];
+                o += c * piece_unit(k, unit0 + u);
             }
-            OutStore<OutT>::store4(P.out, out_row_offset(P, b, kvh, rt * 16 + row, DV) + 4 * c4, o);
+            OutStore<OutT>::store4(P.out, out_at(unit0 + u), L > 0.f ? o / L : (f32x4_t){0.f, 0.f, 0.f, 0.f});
         }
         return;
     }
-    for (int idx = tid; idx < rows_here * (DV / 4); idx += MT) {
-        const int row = idx / (DV / 4), c4 = idx - row * (DV / 4);
+
+    const int G = (UPT == 1 && np > PRE) ? MT / units : 1;  // piece groups
+    const int g = G > 1 ? tid / units : 0, u0 = tid - g * units;
+    f32x4_t pre[UPT][PRE];
+#pragma unroll
+    for (int n = 0; n < UPT; ++n) {
+        const int u = u0 + n * MT;
+#pragma unroll
+        for (int i = 0; i < PRE; ++i)
+            pre[n][i] = (u < units && g < G && g + i * G < np) ? piece_unit(g + i * G, unit0 + u)
+                                                               : (f32x4_t){0.f, 0.f, 0.f, 0.f};
+    }
+
+    // Weights e^{m_w - M} / L of the rows r0 .. r0 + nr - 1.
+    __shared__ float wgt[kMergeTable], lsum[kMergeTable];  // [row][piece]: m, then its weight; l
+    __shared__ float row_inv[16];
+    __shared__ f32x4_t part[UPT == 1 ? kMergeThreads : 1];
+    for (int e = tid; e < nr * np; e += MT) {  // all (m, l) loads in flight at once
+        const int r = e / np;
+        const float *ml = piece_ml(e - r * np, r0 + r);
+        wgt[e] = ml[0];
+        lsum[e] = ml[16];
+    }
+    __syncthreads();
+    const int lanes = np <= 16 ? 16 : 64;  // per row
+    for (int r = tid / lanes; r < nr; r += MT / lanes) {
+        const int l0 = tid & (lanes - 1);
+        float *const w = wgt + r * np, *const ls = lsum + r * np;
         float M = -INFINITY;
-        for (int w = w_first; w <= w_last; ++w) M = fmaxf(M, P.part_ml[piece_of(w) * 32 + row]);
-        float L = 0.f;
-        f32x4_t o = (f32x4_t){0.f, 0.f, 0.f, 0.f};
-#pragma unroll 4
-        for (int w = w_first; w <= w_last; ++w) {
-            const int64_t piece = piece_of(w);
-            const float c = __expf(P.part_ml[piece * 32 + row] - M);
-            L += c * P.part_ml[piece * 32 + 16 + row];
-            o += c * *reinterpret_cast<const f32x4_t *>(P.part_o + (piece * 16 + row) * DV + 4 * c4);
+        for (int k = l0; k < np; k += lanes) M = fmaxf(M, w[k]);
+        M = row16_combine(M, [](float x, float y) { return fmaxf(x, y); });
+        if (lanes == 64) {
+            M = fmaxf(M, __shfl_xor(M, 16, 64));
+            M = fmaxf(M, __shfl_xor(M, 32, 64));
         }
-        const f32x4_t res = L > 0.f ? o / L : (f32x4_t){0.f, 0.f, 0.f, 0.f};
-        OutStore<OutT>::store4(P.out, out_row_offset(P, b, kvh, rt * 16 + row, DV) + 4 * c4, res);
+        float L = 0.f;
+        for (int k = l0; k < np; k += lanes) {
+            const float c = __expf(w[k] - M);
+            w[k] = c;
+            L += c * ls[k];
+        }
+        L = row16_combine(L, [](float x, float y) { return x + y; });
+        if (lanes == 64) {
+            L += __shfl_xor(L, 16, 64);
+            L += __shfl_xor(L, 32, 64);
+        }
+        if (l0 == 0) row_inv[r] = L > 0.f ? 1.f / L : 0.f;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int n = 0; n < UPT; ++n) {
+        const int u = u0 + n * MT;
+        f32x4_t o = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+        if (u < units && g < G) {
+            const int r = (unit0 + u) / UPR - r0;
+            const float *const w = wgt + r * np;
+#pragma unroll
+            for (int i = 0; i < PRE; ++i)
+                if (g + i * G < np) o += w[g + i * G] * pre[n][i];
+#pragma unroll 4
+            for (int k = g + PRE * G; k < np; k += G) o += w[k] * piece_unit(k, unit0 + u);
+            o *= row_inv[r];
+        }
+        if (G > 1) {  // (UPT == 1)
+            part[tid] = o;
+            __syncthreads();
+            if (g == 0)
+                for (int i = 1; i < min(G, np); ++i) o += part[i * units + u0];
+        }
+        if (u < units && g == 0) OutStore<OutT>::store4(P.out, out_at(unit0 + u), o);
     }
 }
 
@@ -2192,8 +2236,7 @@ struct KernelPair {
 };
 
 struct MergeFn {
-    KernelFn fn;  // null if unsupported
-    int threads;  // workgroup size
+    KernelFn fn[3];  // one, two and four units per thread of kMergeThreads; null if unsupported
 };
 
 // GQA decode with 16-bit query and caches of element type `dt` (the

@@ -6,12 +6,22 @@ namespace simpler_hip {
 namespace pa {
 namespace {
 
+template <int DV, typename OutT>
+MergeFn merge_set() {  // a tile of 16 rows has 4 DV units
+    if constexpr (DV > 256)
+        return {{pa_merge_kernel<DV, OutT, 1>, pa_merge_kernel<DV, OutT, 2>, pa_merge_kernel<DV, OutT, 4>}};
+    else if constexpr (DV > 128)
+        return {{pa_merge_kernel<DV, OutT, 1>, pa_merge_kernel<DV, OutT, 2>, nullptr}};
+    else
+        return {{pa_merge_kernel<DV, OutT, 1>, nullptr, nullptr}};
+}
+
 template <int DV>
 MergeFn merge_for(int out_dtype) {
     switch (out_dtype) {
-        case SIMPLER_HIP_DT_FLOAT32: return {pa_merge_kernel<DV, float>, merge_threads<DV>()};
-        case SIMPLER_HIP_DT_BFLOAT16: return {pa_merge_kernel<DV, __bf16>, merge_threads<DV>()};
-        case SIMPLER_HIP_DT_FLOAT16: return {pa_merge_kernel<DV, _Float16>, merge_threads<DV>()};
+        case SIMPLER_HIP_DT_FLOAT32: return merge_set<DV, float>();
+        case SIMPLER_HIP_DT_BFLOAT16: return merge_set<DV, __bf16>();
+        case SIMPLER_HIP_DT_FLOAT16: return merge_set<DV, _Float16>();
         default: return MergeFn{};
     }
 }
