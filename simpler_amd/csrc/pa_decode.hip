@@ -126,13 +126,13 @@ Kernels pick_kernel(const SimplerHipPaDecodeArgs *a, bool append = false) {
     return s;
 }
 
-// Default worker count: compute units x the requested workgroups per CU,
-// capped by what the kernel's register footprint allows. Kernels that read K
-// in half lines (plain loads that rely on the L1 to merge the two halves)
-// measured fastest at two waves per CU (512 workers: 112.8 us on the Qwen3-8B
-// bs=32 shape, against 119.2 us with four per CU, whose K streams evict each
-// other's L1 lines). Kernels that read K in whole rows and fp8 caches ask for
-// four (one per SIMD).
+int current_device() {
+    int dev = -1;
+    return hipGetDevice(&dev) == hipSuccess ? dev : -1;
+}
+
+// Default worker count: compute units x the requested workgroups per CU
+// (workers_per_cu), capped by what the kernel's register footprint allows.
 // Without a device (host-only builds and tests) an MI355X is assumed:
 // 256 CUs.
 int wave_slots(KernelFn fn, int threads, int want_per_cu, size_t lds = 0) {
@@ -146,21 +146,16 @@ int wave_slots(KernelFn fn, int threads, int want_per_cu, size_t lds = 0) {
     };
     static std::mutex mu;
     static std::vector<Entry> cache;
-    int dev = -1;
-    if (hipGetDevice(&dev) != hipSuccess) dev = -1;
+    const int dev = current_device();
     std::lock_guard<std::mutex> lk(mu);
     for (const Entry &e : cache)
         if (e.fn == fn && e.device == dev && e.threads == threads && e.want == want_per_cu && e.lds == lds)
             return e.slots;
-    // kWorkersPerCu workgroups per CU, or as many as fit (a 4-wave workgroup
-    // fills a CU at one wave per SIMD). Two 2-wave workers per CU measured
-    // 195.5 us on the speculative-verify shape against 213.9 us with one.
     int per_cu = want_per_cu;
     int cus = 256;
     // Without a device: the kernels use the whole register file of a SIMD
     // (one wave per SIMD, four SIMDs per CU), the MLA kernel most of the LDS.
-    const int fit = 256 / threads;
-    if (fit < per_cu) per_cu = fit > 0 ? fit : 1;
+    if (dev < 0) per_cu = std::max(1, std::min(per_cu, 256 / threads));
     if (dev >= 0) {
         int v = 0;
         if (hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && v > 0) cus = v;
@@ -174,6 +169,37 @@ int wave_slots(KernelFn fn, int threads, int want_per_cu, size_t lds = 0) {
     const int slots = cus * per_cu;
     cache.push_back({fn, dev, threads, want_per_cu, lds, slots});
     return slots;
+}
+
+// Workers per CU of the GQA kernels (wave_slots lowers it to what fits).
+// - K in whole rows through LDS, one row tile: one per SIMD (108.9 us at four,
+//   108.2 at three on the Qwen3-8B bs=32 shape, but 164.5 against 165.5 on
+//   long contexts).
+// - Two-tile waves, whose blocks take twice the math per byte: three (the
+//   verify shape 134.2 us against 142.9 with four).
+// - Waves that keep K and V in registers and read rows of 128 bytes or less
+//   (head dims to 64, fp8 caches): a wave has one block of K and one of V in
+//   flight, 4 KB with 16-token blocks of 64 dims, so the smaller the block
+//   the more waves a CU needs. us per main launch, 37 sequences of 300 to 5000
+//   tokens, 8 kv heads of 64 dims, at 2 / 4 / 6 / 8 per CU: 16-token blocks
+//   104.4 / 60.1 / 43.5 / 36.2; 32: 71.8 / 42.3 / 34.5 / 36.3; 64: 55.9 / 37.2
+//   / 37.8 / 37.1; 128: 58.6 / 37.8 / 49.5 / 43.3. fp8 (32 sequences to 8192)
+//   at 3 / 4 / 8: 101.4 / 79.6 / 54.2; 66.8 / 54.9 / 57.8; 54.2 / 57.1 / 58.2;
+//   59.1 / 56.5 / 57.6.
+// - 256-dim heads: two (four and more measured 2-8% slower), but four where a
+//   block exceeds the registers and runs unpipelined (151.6 against 170.7).
+// - Sibling waves (several row tiles per worker): two workgroups.
+// A plan made without a device (which can launch nothing) reports nominal
+// counts that do not depend on the block size.
+int workers_per_cu(const SimplerHipPaDecodeArgs *a, const KernelPair &k, KernelFn main, bool pair) {
+    if (pair) return kWorkersThreePerCu;
+    if (main != k.main) return kWorkersPerCu;
+    if (k.klds) return kWorkersPerSimdCu;
+    const int bs = a->block_size;
+    if (current_device() < 0) return a->kv_format == SIMPLER_HIP_KV_FP8_E4M3 ? kWorkersThreePerCu : kWorkersPerCu;
+    if (a->kv_format == SIMPLER_HIP_KV_FP8_E4M3) return bs <= 16 ? 8 : bs == 64 ? 3 : 4;
+    if (a->head_dim_k <= 64) return bs <= 16 ? 8 : bs <= 32 ? 6 : 4;
+    return bs * a->head_dim_k > 16384 ? 4 : kWorkersPerCu;
 }
 
 Plan make_plan(const SimplerHipPaDecodeArgs *a, const KernelPair &k) {  // k: the main kernels of pick_kernel
@@ -215,18 +241,7 @@ Plan make_plan(const SimplerHipPaDecodeArgs *a, const KernelPair &k) {  // k: th
         if (!pair && k.klds && p.tiles_per_worker > 1) p.lds = (size_t)p.tiles_per_worker * a->block_size * 256;
         p.groups = 1;
         p.row_groups = (p.row_tiles + p.tiles_per_worker - 1) / p.tiles_per_worker;
-        // One worker per SIMD when K is read in whole rows (through LDS); three
-        // per CU for fp8 caches and for two-tile waves, whose blocks take
-        // twice the math per byte (same-box medians at 768 against 1024
-        // workers: fp8 57.4 against 58.7 us, the verify shape 134.2 against
-        // 142.9; the single-tile kernel 108.2 against 108.9 on cfg2 but 165.5
-        // against 164.5 on cfg3, so it keeps four); two per CU when K is read
-        // in half lines, whose plain loads rely on the L1 merging the two
-        // halves and evict each other at four.
-        const bool fp8_kv = a->kv_format == SIMPLER_HIP_KV_FP8_E4M3;
-        const int per_cu = (fp8_kv || pair) ? kWorkersThreePerCu
-                           : (k.klds && p.main == k.main) ? kWorkersPerSimdCu
-                                                          : kWorkersPerCu;
+        const int per_cu = workers_per_cu(a, k, p.main, pair);
         p.workers = a->num_workers > 0 ? a->num_workers : wave_slots(p.main, p.threads, per_cu, p.lds);
         // Work lists (the tiles of a batch shared out among them, rotating with
         // the batch). 16-bit caches: one list per tile of a batch when the
