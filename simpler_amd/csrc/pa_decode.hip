@@ -188,18 +188,32 @@ int wave_slots(KernelFn fn, int threads, int want_per_cu, size_t lds = 0) {
 //   59.1 / 56.5 / 57.6.
 // - 256-dim heads: two (four and more measured 2-8% slower), but four where a
 //   block exceeds the registers and runs unpipelined (151.6 against 170.7).
-// - Sibling waves (several row tiles per worker): two workgroups.
+// - Sibling waves (several row tiles per worker): the same by waves, since
+//   the siblings' loads meet in the caches. us per main launch, 16 sequences of
+//   4 kv heads (122 MB), 2 / 3 / 4 tiles, against two, one and one workgroups
+//   per CU: 64 dims x 16 tokens 35.5 / 48.7 / 59.5 against 63.0 / 108 / 115,
+//   x 32 31.5 / 42.3 / 51.9 against 44.0 / 73.3 / 75.2; 128 dims x 16 tokens,
+//   3 / 4 tiles, 35.7 / 40.0 against 49.9 / 52.6 (at 64 and 128 tokens one
+//   workgroup is best); fp8, 2 tiles, 16 / 32 / 64 tokens 42.7 / 35.3 / 34.1
+//   against 75.1 / 51.4 / 41.0.
 // A plan made without a device (which can launch nothing) reports nominal
 // counts that do not depend on the block size.
-int workers_per_cu(const SimplerHipPaDecodeArgs *a, const KernelPair &k, KernelFn main, bool pair) {
+int workers_per_cu(const SimplerHipPaDecodeArgs *a, const KernelPair &k, const Plan &p, bool pair) {
     if (pair) return kWorkersThreePerCu;
-    if (main != k.main) return kWorkersPerCu;
+    const int bs = a->block_size, d = a->head_dim_k, tiles = p.tiles_per_worker;
+    const bool fp8 = a->kv_format == SIMPLER_HIP_KV_FP8_E4M3, nominal = current_device() < 0;
+    if (tiles > 1) {
+        if (nominal) return kWorkersPerCu;
+        const int waves = (d <= 64 || fp8) ? (bs <= 16 ? 12 : bs <= 32 ? 9 : bs <= 64 ? 6 : 4)
+                          : d <= 128       ? (bs <= 16 ? 8 : bs <= 32 ? 6 : 4)
+                                           : 4;
+        return std::max(1, waves / tiles);
+    }
     if (k.klds) return kWorkersPerSimdCu;
-    const int bs = a->block_size;
-    if (current_device() < 0) return a->kv_format == SIMPLER_HIP_KV_FP8_E4M3 ? kWorkersThreePerCu : kWorkersPerCu;
-    if (a->kv_format == SIMPLER_HIP_KV_FP8_E4M3) return bs <= 16 ? 8 : bs == 64 ? 3 : 4;
-    if (a->head_dim_k <= 64) return bs <= 16 ? 8 : bs <= 32 ? 6 : 4;
-    return bs * a->head_dim_k > 16384 ? 4 : kWorkersPerCu;
+    if (nominal) return fp8 ? kWorkersThreePerCu : kWorkersPerCu;
+    if (fp8) return bs <= 16 ? 8 : bs == 64 ? 3 : 4;
+    if (d <= 64) return bs <= 16 ? 8 : bs <= 32 ? 6 : 4;
+    return bs * d > 16384 ? 4 : kWorkersPerCu;
 }
 
 Plan make_plan(const SimplerHipPaDecodeArgs *a, const KernelPair &k) {  // k: the main kernels of pick_kernel
@@ -241,7 +255,7 @@ Plan make_plan(const SimplerHipPaDecodeArgs *a, const KernelPair &k) {  // k: th
         if (!pair && k.klds && p.tiles_per_worker > 1) p.lds = (size_t)p.tiles_per_worker * a->block_size * 256;
         p.groups = 1;
         p.row_groups = (p.row_tiles + p.tiles_per_worker - 1) / p.tiles_per_worker;
-        const int per_cu = workers_per_cu(a, k, p.main, pair);
+        const int per_cu = workers_per_cu(a, k, p, pair);
         p.workers = a->num_workers > 0 ? a->num_workers : wave_slots(p.main, p.threads, per_cu, p.lds);
         // Work lists (the tiles of a batch shared out among them, rotating with
         // the batch). 16-bit caches: one list per tile of a batch when the
