@@ -92,7 +92,8 @@ typedef struct SimplerHipPaDecodeArgs {
     float scale;
     int32_t causal;
     /* 0 = one worker wavefront per wave slot of the device; > 0 forces the
-     * number of workers the (tile, KV block) work list is divided among. */
+     * number of workers the (tile, KV block) work list is divided among (and
+     * keeps short contexts on the work list). */
     int32_t num_workers;
     /* SIMPLER_HIP_KV_BF16 (0), SIMPLER_HIP_KV_FP8_E4M3 (1) or SIMPLER_HIP_KV_FP16 (2). */
     int32_t kv_format;
@@ -115,7 +116,9 @@ int simpler_hip_pa_decode_workspace_init(void *workspace, size_t workspace_bytes
 /*
  * Enqueue the decode on `stream`: the fused kernel (one wavefront per worker,
  * each over an equal slice of the flattened (tile, KV block) work), then the
- * small kernel that merges tiles cut between workers. `workspace` must be at
+ * small kernel that merges tiles cut between workers; or, where num_workers is
+ * 0 and the block table is too narrow for a long context, one kernel with one
+ * workgroup per tile. `workspace` must be at
  * least simpler_hip_pa_decode_workspace_size(args) bytes, 256-byte aligned,
  * initialised once with simpler_hip_pa_decode_workspace_init, and not shared by
  * calls that may run concurrently. Returns 0 or a negative SIMPLER_HIP_ERR_*
@@ -126,7 +129,8 @@ int simpler_hip_pa_decode(const SimplerHipPaDecodeArgs *args, void *workspace, s
 /* The two kernels of simpler_hip_pa_decode, separately (measurement: lets a
  * caller put timing events between them). Running MAIN then MERGE on one
  * stream is exactly simpler_hip_pa_decode; MERGE reads what MAIN wrote to the
- * workspace, so it must follow a MAIN with the same args and workspace. */
+ * workspace, so it must follow a MAIN with the same args and workspace (and
+ * launches nothing where MAIN is the whole decode). */
 enum { SIMPLER_HIP_PHASE_MAIN = 1, SIMPLER_HIP_PHASE_MERGE = 2 };
 int simpler_hip_pa_decode_phase(const SimplerHipPaDecodeArgs *args, void *workspace, size_t workspace_bytes,
                                 void *stream, int phases);
@@ -180,9 +184,9 @@ int simpler_hip_pa_decode_noalloc(const SimplerHipPaDecodeArgs *args, void *stre
  * by simpler_hip_pa_decode. q_len <= 16; bf16 and fp16 caches (not fp8).
  * The append is fused into the decode's two launches where each worker runs
  * one row tile; where the decode gives a worker several row tiles (GQA with
- * more than 16 query rows per kv head) and for MLA, it runs as a launch of
- * its own ahead of them, which measured faster there. Both forms leave the
- * same cache contents.
+ * more than 16 query rows per kv head), for MLA and ahead of the one-kernel
+ * decode of short contexts, it runs as a launch of its own, which measured
+ * faster there. Both forms leave the same cache contents.
  * Same workspace as simpler_hip_pa_decode for these args. A length below
  * q_len or above max_blocks_per_seq*block_size is reported by
  * simpler_hip_pa_decode_check as BAD_LENGTH: the new tokens are still placed
@@ -208,7 +212,7 @@ int simpler_hip_pa_decode_append(const SimplerHipPaDecodeArgs *args, const void 
  * paged attention; in the reference the prelude and the cache write are
  * phase 0 of the fused attention task, paged_attention_cce/kernel/
  * fai_body.hpp:199-230). Three launches on `stream`: the prelude (its query
- * rows into the workspace), then the decode's two. Results and cache
+ * rows into the workspace), then the decode's. Results and cache
  * contents equal, bit for bit, simpler_hip_qk_norm_rope_append per token
  * (position context_lens[b] - q_len + i, slot from the block table) followed
  * by simpler_hip_pa_decode on its query.

@@ -26,6 +26,9 @@ SOURCES = [
     CSRC / "pa_kernels_gqa_bf16_append.hip",
     CSRC / "pa_kernels_gqa_f16_append.hip",
     CSRC / "pa_kernels_fp8.hip",
+    CSRC / "pa_kernels_direct_bf16.hip",
+    CSRC / "pa_kernels_direct_f16.hip",
+    CSRC / "pa_kernels_direct_fp8.hip",
     CSRC / "pa_kernels_mla.hip",
     CSRC / "pa_kernels_merge.hip",
     CSRC / "kv_cache.hip",

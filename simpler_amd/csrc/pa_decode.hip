@@ -29,6 +29,7 @@ using namespace pa;
 constexpr int kZeroOffset = 128;  // workspace bytes [128, 256) are never written after init
 constexpr int kMaxAppendTokens = 16;  // fused append: new tokens per sequence (one per residue mod 16)
 constexpr size_t kMaxZeroPageBytes = 1 << 20;  // larger token strides read the padding tiles as they are
+constexpr int64_t kDirectManyTiles = 128, kDirectTileBytes = 512 << 10, kDirectWaveBytes = 48 << 10;  // direct_waves
 constexpr int kMlaSegTokens = 256;  // MLA: work charged for each sequence a slice starts, in tokens
 
 struct Plan {
@@ -103,6 +104,7 @@ bool v_is_k_prefix(const SimplerHipPaDecodeArgs *a) {
 struct Kernels {
     KernelPair k;
     KernelPair ka;
+    DirectFn direct;
     MergeFn merge;
 };
 
@@ -111,7 +113,10 @@ Kernels pick_kernel(const SimplerHipPaDecodeArgs *a, bool append = false) {
     const int bs = a->block_size, dk = a->head_dim_k, dv = a->head_dim_v, out = a->out_dtype;
     const bool f16 = a->kv_format == SIMPLER_HIP_KV_FP16;
     if (a->kv_format == SIMPLER_HIP_KV_FP8_E4M3) {
-        if (dk == dv && !append) s.k = pick_gqa_fp8(bs, dk, out);  // no fused append for fp8 caches
+        if (dk == dv && !append) {  // no fused append for fp8 caches
+            s.k = pick_gqa_fp8(bs, dk, out);
+            s.direct = pick_direct_fp8(bs, dk, out);
+        }
     } else if (is_mla_shape(a)) {
         // (the kernel's fill offsets use 24-bit multiplies: token rows below 8 MB)
         if (v_is_k_prefix(a) && a->kv_format == SIMPLER_HIP_KV_BF16 && a->k_token_stride * 2 < (1 << 23)) {
@@ -119,6 +124,7 @@ Kernels pick_kernel(const SimplerHipPaDecodeArgs *a, bool append = false) {
         }
     } else if (dk == dv) {
         s.k = f16 ? pick_gqa_f16(bs, dk, out) : pick_gqa_bf16(bs, dk, out);
+        s.direct = f16 ? pick_direct_f16(bs, dk, out) : pick_direct_bf16(bs, dk, out);
         if (append) s.ka = f16 ? pick_gqa_f16_append(bs, dk, out) : pick_gqa_bf16_append(bs, dk, out);
     }
     s.merge = pick_merge(dv, out);
@@ -297,8 +303,54 @@ Plan make_plan(const SimplerHipPaDecodeArgs *a, const KernelPair &k) {  // k: th
     return p;
 }
 
+// Waves per workgroup of the short-context kernels (pa_kernels_direct.h), or 0
+// where the work lists run: the caller forced a worker count, or a context may
+// be long (the host knows the table's width, not the lengths). One workgroup
+// per tile saves the merge launch and the work scan, but does not balance
+// lengths, so it is taken where the longest possible tile is short:
+// - with 128 tiles or more, up to 512 KB of K and V per tile (1024 tokens of
+//   128 dims), for kernels that keep few bytes in flight (head dims to 64, fp8
+//   caches) up to 256 KB. us per step against the work lists, 8 kv heads, D =
+//   128, 128-token blocks: 32 sequences of 100-500 tokens 12.0 against 17.2,
+//   of 200-1000 19.1 against 22.7; 130 of 512 54.0 against 57.4; 256 of
+//   200-1000 113 against 125; 256 of 16-40 21.6 against 30.5. At twice the
+//   limit, 130 of 100-2048, 118 against 110. Every row tile of a kv head reads
+//   K and V again, so its tiles together stay within 768 KB (32 x 4 kv heads of
+//   64 rows, 100-500 tokens 20.7 against 23.5, 200-1000 34.4 against 27.8).
+// - with fewer tiles, where each wave takes one block at most, or 48 KB:
+//   2 sequences of 512 tokens and 1 kv head 7.9 against 10.6, of 16-40 tokens
+//   in 16-token blocks 5.0 against 8.3; at two 64 KB blocks per wave 16.2
+//   against 13.5.
+// Waves per tile: enough for workers_per_cu waves on every CU, at least four.
+int direct_waves(const SimplerHipPaDecodeArgs *a, const Kernels &s, const Plan &p) {
+    if (!s.direct.fn || a->num_workers > 0) return 0;
+    const bool fp8 = a->kv_format == SIMPLER_HIP_KV_FP8_E4M3;
+    const int64_t blocks = a->max_blocks_per_seq;
+    const int64_t block_bytes = (int64_t)a->block_size * 2 * a->head_dim_k * (fp8 ? 1 : 2);
+    const int64_t tiles = std::max<int64_t>((int64_t)a->batch * a->num_kv_heads * p.row_tiles, 1);
+    if (blocks * block_bytes > kDirectTileBytes) return 0;
+    Plan one = p;
+    one.tiles_per_worker = 1;
+    const int64_t want = 256 * (int64_t)std::max(kWorkersPerSimdCu, workers_per_cu(a, s.k, one, false));
+    const int64_t waves = std::min<int64_t>({(want + tiles - 1) / tiles, s.direct.max_waves, blocks});
+    const int64_t per_wave = (blocks + waves - 1) / waves;
+    const bool narrow = fp8 || a->head_dim_k <= 64;
+    if (!narrow && p.row_tiles > 1 && blocks * block_bytes * p.row_tiles > kDirectTileBytes * 3 / 2) return 0;
+    if (tiles >= kDirectManyTiles ? narrow && blocks * block_bytes > kDirectTileBytes / 2
+                                  : per_wave > 1 && per_wave * block_bytes > kDirectWaveBytes)
+        return 0;
+    return (int)waves;
+}
+
+// Writes the error word into the host's mirror, after everything before it on
+// the stream.
+__global__ void mirror_kernel(const unsigned *flag, unsigned *mirror) {
+    __hip_atomic_store(mirror, *flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // The merge's launch: workgroups per tile (grid y), each with `units` of the
-// tile's 16-byte units. A tile is cut into about workers / tiles + 1 pieces.
+// tile's 16-byte units. A tile is cut into about workers / tiles + 1 pieces,
+// at most one per block.
 // It is shared out among workgroups (down to 8 units, a 128-byte line, each)
 // until a thread has one unit and reads kMergeAhead of its pieces at most,
 // as long as the grid stays within kMergeGrid workgroups: with more, every
@@ -317,7 +369,8 @@ MergePlan plan_merge(const MergeFn &m, const SimplerHipPaDecodeArgs *a, const Pl
     const int64_t all = (int64_t)std::min(16, p.rows) * (a->head_dim_v / 4);
     const int64_t lists = (int64_t)a->batch * a->num_kv_heads;
     const int64_t tiles = std::max<int64_t>(lists * p.row_tiles, 1);
-    const int64_t pieces = p.workers / std::max<int64_t>(lists * p.row_groups, 1) + 1;
+    const int64_t pieces = std::min<int64_t>(p.workers / std::max<int64_t>(lists * p.row_groups, 1) + 1,
+                                             a->max_blocks_per_seq);
     MergePlan r{};
     int64_t units = all, groups = 1;
     while (units >= 16 && tiles * groups * 2 <= kMergeGrid &&
@@ -455,6 +508,18 @@ int pa_decode_launch(const SimplerHipPaDecodeArgs *a, void *workspace, size_t wo
     P.v_new = (const uint16_t *)v_new;
 
     const int64_t tiles = (int64_t)a->batch * a->num_kv_heads * plan.row_tiles;
+    if (const int waves = append ? 0 : direct_waves(a, s, plan)) {
+        if (phases & SIMPLER_HIP_PHASE_MAIN) {
+            hipLaunchKernelGGL(s.direct.fn, dim3((unsigned)tiles), dim3(64u * waves),
+                               (unsigned)(waves * s.direct.wave_lds), (hipStream_t)stream, P);
+            if (hipGetLastError() != hipSuccess) return SIMPLER_HIP_ERR_LAUNCH;
+        }
+        if (P.err_mirror) {
+            hipLaunchKernelGGL(mirror_kernel, dim3(1), dim3(1), 0, (hipStream_t)stream, P.error_flag, P.err_mirror);
+            if (hipGetLastError() != hipSuccess) return SIMPLER_HIP_ERR_LAUNCH;
+        }
+        return SIMPLER_HIP_OK;
+    }
     const MergePlan merge = plan_merge(s.merge, a, plan);
     P.merge_units = merge.units;
     if (phases & SIMPLER_HIP_PHASE_MAIN) {
@@ -503,7 +568,7 @@ extern "C" int simpler_hip_pa_decode_append(const SimplerHipPaDecodeArgs *a, con
         const Kernels s = pick_kernel(a);
         if (s.k.main) {
             const Plan plan = make_plan(a, s.k);
-            if (plan.tiles_per_worker > 1 || s.k.mla) {
+            if (plan.tiles_per_worker > 1 || s.k.mla || direct_waves(a, s, plan)) {
                 if (!workspace || workspace_bytes < plan.total || ((uintptr_t)workspace & 255))
                     return SIMPLER_HIP_ERR_WORKSPACE;
                 if (a->batch == 0) return SIMPLER_HIP_OK;

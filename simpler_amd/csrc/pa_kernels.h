@@ -2235,6 +2235,13 @@ struct KernelPair {
     KernelFn main_pair = nullptr;  // one wave per worker running two row tiles (K through LDS), or null
 };
 
+// Short-context decode (pa_kernels_direct.h): one workgroup of up to
+// max_waves waves per 16-row tile, wave_lds bytes of dynamic LDS each.
+struct DirectFn {
+    KernelFn fn;  // null if unsupported
+    int max_waves, wave_lds;
+};
+
 struct MergeFn {
     KernelFn fn[3];  // one, two and four units per thread of kMergeThreads; null if unsupported
 };
@@ -2248,6 +2255,10 @@ KernelPair pick_gqa_bf16_append(int bs, int d, int out_dtype);
 KernelPair pick_gqa_f16_append(int bs, int d, int out_dtype);
 // GQA decode with fp8 E4M3FN caches (bf16 query), Dk == Dv == 128.
 KernelPair pick_gqa_fp8(int bs, int d, int out_dtype);
+// The short-context kernels of the above.
+DirectFn pick_direct_bf16(int bs, int d, int out_dtype);
+DirectFn pick_direct_f16(int bs, int d, int out_dtype);
+DirectFn pick_direct_fp8(int bs, int d, int out_dtype);
 // MLA (Dk 576, Dv 512, V a prefix of K), bf16.
 KernelPair pick_mla(int bs, int out_dtype);
 // The split merge for output width dv.

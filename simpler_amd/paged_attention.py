@@ -354,7 +354,7 @@ def paged_attention_decode_prelude(
     num_workers: int = 0,
 ) -> torch.Tensor:
     """Decode prelude, KV append and decode in one call
-    (``simpler_hip_pa_decode_prelude``: the prelude's launch, then the decode's two).
+    (``simpler_hip_pa_decode_prelude``: the prelude's launch, then the decode's).
 
     From the fp32 projections ``q_proj`` ``[B, (q_len,) Hq, 128]`` and ``k_proj``
     / ``v_proj`` ``[B, (q_len,) Hkv, 128]``: q and k are RoPE(RMSnorm(proj *

@@ -1,0 +1,83 @@
+"""The short-context decode (one workgroup per tile, no merge launch) at the
+edges of its shapes: fewer blocks than waves, one more, a last partial block,
+empty contexts, row tiles past the first, causal rows, the table widths on
+both sides of the rule that selects it, and its error reports."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from oracle import pa_oracle as po
+from simpler_amd import paged_attention as pa
+from simpler_amd.workloads import make_custom_case, quantize_kv_fp8
+from tests.pa_helpers import assert_close, oracle_numpy
+
+pytestmark = pytest.mark.gpu
+
+
+def run(case, device, **kw):
+    d = case.to(device)
+    if d.k_scale is not None:
+        kw.update(k_scale=d.k_scale, v_scale=d.v_scale)
+    out = pa.paged_attention_decode(d.query, d.key_cache, d.value_cache, d.block_table, d.context_lens,
+                                    scale=case.scale, causal=case.config.causal, **kw)
+    torch.cuda.synchronize(device)
+    return out.cpu().numpy()
+
+
+# (heads, kv heads, dim, block, lengths, q_len, table width in blocks)
+@pytest.mark.parametrize("hq,hkv,dim,bs,lens,q_len,width", [
+    (4, 1, 16, 16, [1, 0, 16, 17, 255, 256], 1, 16),      # one block per wave at most
+    (16, 2, 64, 16, [0, 300, 511], 1, 32),                # two blocks for some waves
+    (8, 8, 128, 128, [512, 385, 1, 0], 1, 4),             # one row, four waves
+    (10, 2, 128, 64, [130, 64], 1, 4),
+    (8, 1, 128, 32, [31, 33, 255], 1, 8),
+    (4, 2, 256, 64, [200, 1], 1, 4),
+    (4, 2, 256, 128, [128, 77], 1, 1),                    # blocks larger than the registers
+    (40, 2, 128, 16, [97, 20], 1, 8),                     # a second row tile of 4 rows
+    (32, 4, 64, 32, [8, 100, 64], 8, 4),                  # causal, four row tiles
+    (32, 32, 64, 64, [1024, 3, 700, 0, 65], 1, 16),       # many tiles: one wave or two each
+    (16, 1, 128, 128, [512, 400], 1, 5),                  # a table one block wider: the work lists
+])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_short_contexts(hq, hkv, dim, bs, lens, q_len, width, dtype, device):
+    print(f"[case] {hq}/{hkv} d{dim} bs{bs} {lens} q{q_len} width {width} {dtype}", flush=True)
+    case = make_custom_case(batch=len(lens), num_heads=hq, kv_heads=hkv, head_dim=dim, block_size=bs, q_len=q_len,
+                            causal=q_len > 1, context_lens=lens, seed=1200 + hq + dim + bs, dtype=dtype,
+                            max_blocks=width)
+    assert_close(run(case, device), oracle_numpy(case), what=f"d{dim} bs{bs}")
+    pa.check_errors(device)
+
+
+@pytest.mark.parametrize("bs", [16, 32, 64, 128])
+def test_short_fp8_contexts(bs, device):
+    case = make_custom_case(batch=3, num_heads=8, kv_heads=2, head_dim=128, block_size=bs, context_lens=[5, 130, 256],
+                            seed=1300 + bs)
+    case.key_cache, case.k_scale = quantize_kv_fp8(case.key_cache, pow2=False)
+    case.value_cache, case.v_scale = quantize_kv_fp8(case.value_cache, pow2=False)
+    k = po.dequantize_kv(case.key_cache.view(torch.uint8).numpy(), case.k_scale.numpy())
+    v = po.dequantize_kv(case.value_cache.view(torch.uint8).numpy(), case.v_scale.numpy())
+    ref = po.paged_attention_decode(case.query.float().numpy(), k, v, case.block_table.numpy(),
+                                    case.context_lens.numpy(), case.scale)
+    assert_close(run(case, device), ref, what=f"fp8 bs{bs}")
+
+
+def test_errors_are_reported(device):
+    case = make_custom_case(batch=2, num_heads=8, kv_heads=2, head_dim=128, block_size=64, context_lens=[100, 128],
+                            seed=1400, max_blocks=2)
+    base = run(case, device)
+    pa.check_errors(device)
+    case.context_lens[1] = 129  # past the table: clamped to 128 and reported
+    got = run(case, device)
+    assert (got == base).all()
+    with pytest.raises(pa.PagedAttentionError) as e:
+        pa.check_errors(device)
+    assert e.value.rc == -7
+    case.context_lens[1] = 128
+    case.block_table[0, 1] = 99  # outside the pool: skipped and reported
+    run(case, device)
+    with pytest.raises(pa.PagedAttentionError) as e:
+        pa.check_errors(device)
+    assert e.value.rc == -6
+    pa.check_errors(device)
