@@ -211,8 +211,8 @@ int simpler_hip_pa_decode_append(const SimplerHipPaDecodeArgs *args, const void 
  * layer (simpler_setup/goldens/qwen3_14b_decode.py:207-226, 261-269, then the
  * paged attention; in the reference the prelude and the cache write are
  * phase 0 of the fused attention task, paged_attention_cce/kernel/
- * fai_body.hpp:199-230). Three launches on `stream`: the prelude (its query
- * rows into the workspace), then the decode's. Results and cache
+ * fai_body.hpp:199-230). On `stream`: the prelude's launch (its query rows
+ * into the workspace), then the decode's. Results and cache
  * contents equal, bit for bit, simpler_hip_qk_norm_rope_append per token
  * (position context_lens[b] - q_len + i, slot from the block table) followed
  * by simpler_hip_pa_decode on its query.

@@ -206,6 +206,8 @@ SIGNATURES: dict[str, tuple] = {
 def lib() -> ctypes.CDLL:
     """The loaded native library; raises if it has not been built."""
     global _lib
+    if _lib is not None:
+        return _lib
     with _lock:
         if _lib is not None:
             return _lib

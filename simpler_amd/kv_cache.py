@@ -13,11 +13,12 @@ memory and the stream only, and there is no fallback.
 from __future__ import annotations
 
 import ctypes
+import struct
 
 import torch
 
 from . import _lib
-from .paged_attention import PagedAttentionError
+from .paged_attention import PagedAttentionError, _current_stream
 
 EPS = 1e-6  # the golden's eps (qwen3_14b_decode.py:46)
 
@@ -89,15 +90,60 @@ def kv_append(key: torch.Tensor, value: torch.Tensor | None, slot_mapping: torch
 def launch_append(a: _lib.KvAppendArgs, device: torch.device | None = None, stream: int | None = None) -> None:
     """Enqueue a prepared append (``append_args``) on ``stream`` (default: torch's current stream)."""
     if stream is None:
-        stream = torch.cuda.current_stream(device).cuda_stream
+        stream = (_current_stream(device) if device is not None
+                  else torch.cuda.current_stream(device).cuda_stream)
     rc = _lib.lib().simpler_hip_kv_append(ctypes.byref(a), stream)
     if rc != 0:
         raise PagedAttentionError(rc, "simpler_hip_kv_append")
 
 
+# SimplerHipKvAppendArgs as _lib.KvAppendArgs lays it out
+_APPEND = struct.Struct("@6P10q6i")
+assert _APPEND.size == ctypes.sizeof(_lib.KvAppendArgs)
+
+
+def _plain_append(key, value, slot_mapping, key_cache, value_cache, error_count) -> _lib.KvAppendArgs | None:
+    """``append_args`` where the tensors are as its checks want them, in one pass; None leaves the call to the checks."""
+    try:
+        bf16 = torch.bfloat16
+        tokens, hkv, dk = key.shape
+        nblk, bs, chkv, cdk = key_cache.shape
+        kt, kh, k1 = key.stride()
+        cb, ct, ch, c1 = key_cache.stride()
+        if not (key.dtype is bf16 and key_cache.dtype is bf16 and slot_mapping.dtype is torch.int32 and key.is_cuda
+                and key_cache.is_cuda and slot_mapping.is_cuda and k1 == 1 and c1 == 1 and chkv == hkv and cdk == dk
+                and slot_mapping.shape == (tokens,) and slot_mapping.is_contiguous()):
+            return None
+        vp = vcp = vt = vh = vb = vct = vch = dv = 0
+        if value is not None:
+            vn, vhkv, dv = value.shape
+            vt, vh, v1 = value.stride()
+            vb, vct, vch, vc1 = value_cache.stride()
+            if not (value.dtype is bf16 and value_cache.dtype is bf16 and value.is_cuda and value_cache.is_cuda
+                    and v1 == 1 and vc1 == 1 and vn == tokens and vhkv == hkv
+                    and value_cache.shape == (nblk, bs, hkv, dv)):
+                return None
+            vp, vcp = value.data_ptr(), value_cache.data_ptr()
+        elif value_cache is not None:
+            return None
+        err = 0
+        if error_count is not None:
+            if error_count.dtype is not torch.int32 or not error_count.is_cuda:
+                return None
+            err = error_count.data_ptr()
+        return _lib.KvAppendArgs.from_buffer_copy(_APPEND.pack(
+            key.data_ptr(), vp, slot_mapping.data_ptr(), key_cache.data_ptr(), vcp, err, kt, kh, vt, vh, cb, ct, ch,
+            vb, vct, vch, tokens, hkv, dk, dv, bs, nblk))
+    except (AttributeError, TypeError, ValueError, struct.error):
+        return None
+
+
 def append_args(key: torch.Tensor, value: torch.Tensor | None, slot_mapping: torch.Tensor, key_cache: torch.Tensor,
                 value_cache: torch.Tensor | None, error_count: torch.Tensor | None = None) -> _lib.KvAppendArgs:
     """Validate the tensors of an append and fill the C ``SimplerHipKvAppendArgs``."""
+    a = _plain_append(key, value, slot_mapping, key_cache, value_cache, error_count)
+    if a is not None:
+        return a
     _dev(key, "key", torch.bfloat16)
     _dev(slot_mapping, "slot_mapping", torch.int32)
     _dev(key_cache, "key_cache", torch.bfloat16)
@@ -157,7 +203,8 @@ def launch_prelude(a: _lib.QkNormRopeAppendArgs, device: torch.device | None = N
                    stream: int | None = None) -> None:
     """Enqueue a prepared prelude (``prelude_args``) on ``stream`` (default: torch's current stream)."""
     if stream is None:
-        stream = torch.cuda.current_stream(device).cuda_stream
+        stream = (_current_stream(device) if device is not None
+                  else torch.cuda.current_stream(device).cuda_stream)
     rc = _lib.lib().simpler_hip_qk_norm_rope_append(ctypes.byref(a), stream)
     if rc != 0:
         raise PagedAttentionError(rc, "simpler_hip_qk_norm_rope_append")

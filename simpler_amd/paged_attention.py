@@ -16,6 +16,7 @@ from __future__ import annotations
 
 import ctypes
 import math
+import struct
 import threading
 
 import torch
@@ -64,7 +65,12 @@ class _Workspace:
     def __init__(self) -> None:
         self._mu = threading.Lock()
         self._buf: dict[tuple[int, int], torch.Tensor] = {}
+        self._addr: dict[tuple[int, int], tuple[int, int]] = {}
         self._retired: list[torch.Tensor] = []
+
+    def peek(self, idx: int, stream: int) -> tuple[int, int]:
+        """Address and bytes of the buffer of a device and stream, or (0, 0) before its first use."""
+        return self._addr.get((idx, stream), (0, 0))
 
     def get(self, device: torch.device, nbytes: int, stream: int) -> torch.Tensor:
         idx = device.index if device.index is not None else torch.cuda.current_device()
@@ -83,6 +89,7 @@ class _Workspace:
                 if buf is not None:
                     self._retired.append(buf)  # a captured graph may still use it
                 self._buf[key] = new
+                self._addr[key] = (new.data_ptr(), new.numel())
                 buf = new
             return buf
 
@@ -99,6 +106,56 @@ def _check(t: torch.Tensor, name: str, dtype: torch.dtype, ndims: tuple[int, ...
         raise ValueError(f"{name} must be {dtype}, got {t.dtype}")
     if t.dim() not in ndims:
         raise ValueError(f"{name} must have {ndims} dims, got shape {tuple(t.shape)}")
+
+
+# SimplerHipPaDecodeArgs as _lib.PaDecodeArgs lays it out
+_ARGS = struct.Struct("@6P6q10if3i2P")
+assert _ARGS.size == ctypes.sizeof(_lib.PaDecodeArgs)
+
+
+def _plain_args(query, key_cache, value_cache, block_table, context_lens, out, scale, causal, num_workers, k_scale,
+                v_scale) -> _lib.PaDecodeArgs | None:
+    """``make_args`` where everything is as its checks want it, in one pass over
+    the tensors' attributes and one packing (a small decode takes the device
+    about as long as the call takes the host); None leaves the call to the
+    checks, which name what is wrong."""
+    try:
+        qs, (nblk, bs, hkv, dk), (vnb, vbs, vhkv, dv) = query.shape, key_cache.shape, value_cache.shape
+        qt, kt, ot = query.dtype, key_cache.dtype, out.dtype
+        if len(qs) == 3:
+            (batch, hq, qd), q_len = qs, 1
+        else:
+            batch, q_len, hq, qd = qs
+        if kt is qt and (qt is torch.bfloat16 or qt is torch.float16):
+            fmt, kp, vp = (KV_BF16 if qt is torch.bfloat16 else KV_FP16), 0, 0
+            if k_scale is not None or v_scale is not None:
+                return None
+        elif kt in _FP8_DTYPES and qt is torch.bfloat16:
+            fmt, kp, vp = KV_FP8_E4M3, k_scale.data_ptr(), v_scale.data_ptr()
+            for t in (k_scale, v_scale):
+                if t.dtype is not torch.float32 or t.shape != (nblk, hkv) or not t.is_cuda or not t.is_contiguous():
+                    return None
+        else:
+            return None
+        tb, width = block_table.shape
+        kb, ktk, kh, k1 = key_cache.stride()
+        vb, vtk, vh, v1 = value_cache.stride()
+        if not (
+            value_cache.dtype is kt and (ot is torch.float32 or ot is qt) and qd == dk
+            and vnb == nblk and vbs == bs and vhkv == hkv and k1 == 1 and v1 == 1
+            and out.shape == (*qs[:-1], dv) and tb == batch and context_lens.shape == (batch,)
+            and block_table.dtype is torch.int32 and context_lens.dtype is torch.int32
+            and query.is_cuda and key_cache.is_cuda and value_cache.is_cuda and block_table.is_cuda
+            and context_lens.is_cuda and out.is_cuda and query.is_contiguous() and out.is_contiguous()
+            and block_table.is_contiguous() and context_lens.is_contiguous()
+        ):
+            return None
+        return _lib.PaDecodeArgs.from_buffer_copy(_ARGS.pack(
+            query.data_ptr(), key_cache.data_ptr(), value_cache.data_ptr(), block_table.data_ptr(),
+            context_lens.data_ptr(), out.data_ptr(), kb, ktk, kh, vb, vtk, vh, batch, q_len, hq, hkv, dk, dv, bs,
+            width, nblk, _OUT_DTYPES[ot], scale, 1 if causal else 0, num_workers, fmt, kp, vp))
+    except (AttributeError, TypeError, ValueError, struct.error, OverflowError):
+        return None
 
 
 def make_args(
@@ -122,6 +179,10 @@ def make_args(
     ``[num_blocks, num_kv_heads]``: element (blk, t, h, d) stands for
     ``float(cache[blk, t, h, d]) * scale[blk, h]``.
     """
+    plain = _plain_args(query, key_cache, value_cache, block_table, context_lens, out, scale, causal, num_workers,
+                        k_scale, v_scale)
+    if plain is not None:
+        return plain
     fp8 = key_cache.dtype in _FP8_DTYPES
     fp16 = query.dtype == torch.float16
     kv_dtype = key_cache.dtype if fp8 else (torch.float16 if fp16 else torch.bfloat16)
@@ -188,6 +249,14 @@ def make_args(
 
 PHASE_MAIN, PHASE_MERGE = 1, 2
 
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)  # the stream's address without a Stream object
+
+
+def _current_stream(device: torch.device) -> int:
+    if _raw_stream is not None and device.index is not None:
+        return _raw_stream(device.index)
+    return torch.cuda.current_stream(device).cuda_stream
+
 
 def launch(args: _lib.PaDecodeArgs, device: torch.device, stream: int | None = None,
            phases: int = PHASE_MAIN | PHASE_MERGE, key_new: torch.Tensor | None = None,
@@ -203,36 +272,50 @@ def launch(args: _lib.PaDecodeArgs, device: torch.device, stream: int | None = N
     """
     lib = _lib.lib()
     if stream is None:
-        stream = torch.cuda.current_stream(device).cuda_stream
+        stream = _current_stream(device)
+    both = phases == PHASE_MAIN | PHASE_MERGE
+    if prelude is not None:
+        what = "simpler_hip_pa_decode_prelude"
+
+        def call(ws: int, nbytes: int) -> int:
+            return lib.simpler_hip_pa_decode_prelude(ctypes.byref(args), ctypes.byref(prelude), ws, nbytes, stream)
+    elif key_new is not None:
+        what = "simpler_hip_pa_decode_append"
+
+        def call(ws: int, nbytes: int) -> int:
+            return lib.simpler_hip_pa_decode_append(ctypes.byref(args), key_new.data_ptr(),
+                                                    value_new.data_ptr() if value_new is not None else None, ws,
+                                                    nbytes, stream)
+    else:
+        what = "simpler_hip_pa_decode"
+
+        def call(ws: int, nbytes: int) -> int:
+            if both:
+                return lib.simpler_hip_pa_decode(ctypes.byref(args), ws, nbytes, stream)
+            return lib.simpler_hip_pa_decode_phase(ctypes.byref(args), ws, nbytes, stream, phases)
+    if both and device.index is not None:
+        # The stream's buffer is nearly always large enough, and the call itself
+        # says if not. Whatever else it refuses is left to the checks below.
+        ws_ptr, ws_bytes = _WORKSPACE.peek(device.index, stream or 0)
+        if ws_ptr:
+            rc = call(ws_ptr, ws_bytes)
+            if rc == 0:
+                return
+            if rc == -5:  # launched in part: not to be tried again
+                raise PagedAttentionError(rc, what)
     size_of = (lib.simpler_hip_pa_decode_prelude_workspace_size if prelude is not None
                else lib.simpler_hip_pa_decode_workspace_size)
     need = size_of(ctypes.byref(args))
     if need == 0:
         raise PagedAttentionError(-1)
     ws = _WORKSPACE.get(device, need, stream)
-    if prelude is not None:
-        if phases != PHASE_MAIN | PHASE_MERGE:
-            raise ValueError("the prelude entry runs both phases")
-        rc = lib.simpler_hip_pa_decode_prelude(ctypes.byref(args), ctypes.byref(prelude), ws.data_ptr(), ws.numel(),
-                                               stream)
-        if rc != 0:
-            raise PagedAttentionError(rc, "simpler_hip_pa_decode_prelude")
-        return
-    if key_new is not None:
-        if phases != PHASE_MAIN | PHASE_MERGE:
-            raise ValueError("the fused append runs both phases")
-        rc = lib.simpler_hip_pa_decode_append(ctypes.byref(args), key_new.data_ptr(),
-                                              value_new.data_ptr() if value_new is not None else None,
-                                              ws.data_ptr(), ws.numel(), stream)
-        if rc != 0:
-            raise PagedAttentionError(rc, "simpler_hip_pa_decode_append")
-        return
-    if phases == PHASE_MAIN | PHASE_MERGE:
-        rc = lib.simpler_hip_pa_decode(ctypes.byref(args), ws.data_ptr(), ws.numel(), stream)
-    else:
-        rc = lib.simpler_hip_pa_decode_phase(ctypes.byref(args), ws.data_ptr(), ws.numel(), stream, phases)
+    if prelude is not None and not both:
+        raise ValueError("the prelude entry runs both phases")
+    if key_new is not None and not both:
+        raise ValueError("the fused append runs both phases")
+    rc = call(ws.data_ptr(), ws.numel())
     if rc != 0:
-        raise PagedAttentionError(rc)
+        raise PagedAttentionError(rc, what)
 
 
 def append_tensors(args: _lib.PaDecodeArgs, query: torch.Tensor, key_cache: torch.Tensor,
@@ -387,6 +470,57 @@ def prelude_args(q_proj: torch.Tensor, k_proj: torch.Tensor, v_proj: torch.Tenso
                  num_workers: int = 0) -> tuple[_lib.PaDecodeArgs, _lib.DecodePreludeArgs]:
     """The C decode args and prelude args of ``paged_attention_decode_prelude``,
     for repeated ``launch(args, device, prelude=pre)``; checks the tensors."""
+    args = _plain_prelude(q_proj, k_proj, v_proj, inv_rms, q_norm_weight, k_norm_weight, rope_cos, rope_sin, key_cache,
+                          value_cache, block_table, context_lens, out, scale, causal, num_workers)
+    if args is None:
+        args = _checked_prelude(q_proj, k_proj, v_proj, inv_rms, q_norm_weight, k_norm_weight, rope_cos, rope_sin,
+                                key_cache, value_cache, block_table, context_lens, out, scale, causal, num_workers)
+    pre = _lib.DecodePreludeArgs(
+        q_proj.data_ptr(), k_proj.data_ptr(), v_proj.data_ptr(), inv_rms.data_ptr(), q_norm_weight.data_ptr(),
+        k_norm_weight.data_ptr(), rope_cos.data_ptr(), rope_sin.data_ptr(), rope_cos.shape[0], float(eps))
+    return args, pre
+
+
+class _ComputedQuery:
+    """Stands in for the bf16 query that the prelude computes: its shape, at
+    q_proj's address (not read)."""
+
+    __slots__ = ("shape", "_ptr")
+    dtype, is_cuda = torch.bfloat16, True
+
+    def __init__(self, q_proj: torch.Tensor) -> None:
+        self.shape, self._ptr = q_proj.shape, q_proj.data_ptr()
+
+    def data_ptr(self) -> int:
+        return self._ptr
+
+    def is_contiguous(self) -> bool:
+        return True
+
+
+def _plain_prelude(q_proj, k_proj, v_proj, inv_rms, q_norm_weight, k_norm_weight, rope_cos, rope_sin, key_cache,
+                   value_cache, block_table, context_lens, out, scale, causal, num_workers):
+    """The decode args of a prelude whose tensors are as the checks want them, else None (as ``_plain_args``)."""
+    try:
+        qs, d = q_proj.shape, q_proj.shape[-1]
+        kv, rope, f32 = (*qs[:-2], key_cache.shape[2], d), rope_cos.shape, torch.float32
+        tokens = qs[0] * (qs[1] if len(qs) == 4 else 1)
+        if len(qs) not in (3, 4) or not (
+            k_proj.shape == kv and v_proj.shape == kv and inv_rms.numel() == tokens and q_norm_weight.shape == (d,)
+            and k_norm_weight.shape == (d,) and len(rope) == 2 and rope[1] == d and rope_sin.shape == rope
+        ):
+            return None
+        for t in (q_proj, k_proj, v_proj, inv_rms, q_norm_weight, k_norm_weight, rope_cos, rope_sin):
+            if t.dtype is not f32 or not t.is_contiguous() or not t.is_cuda:
+                return None
+        return _plain_args(_ComputedQuery(q_proj), key_cache, value_cache, block_table, context_lens, out, scale,
+                           causal, num_workers, None, None)
+    except (AttributeError, TypeError):
+        return None
+
+
+def _checked_prelude(q_proj, k_proj, v_proj, inv_rms, q_norm_weight, k_norm_weight, rope_cos, rope_sin, key_cache,
+                     value_cache, block_table, context_lens, out, scale, causal, num_workers) -> _lib.PaDecodeArgs:
     q4 = q_proj.dim() == 4
     q_len = q_proj.shape[1] if q4 else 1
     batch, hq, d = q_proj.shape[0], q_proj.shape[-2], q_proj.shape[-1]
@@ -412,16 +546,8 @@ def prelude_args(q_proj: torch.Tensor, k_proj: torch.Tensor, v_proj: torch.Tenso
     query_shape = torch.empty(0, dtype=torch.bfloat16, device=q_proj.device).set_(
         q_proj.untyped_storage(), q_proj.storage_offset() * 2, tuple(q_proj.shape),
         tuple(torch.empty(q_proj.shape, device="meta").stride()))
-    args = make_args(query_shape, key_cache, value_cache, block_table, context_lens, out, scale, causal=causal,
+    return make_args(query_shape, key_cache, value_cache, block_table, context_lens, out, scale, causal=causal,
                      num_workers=num_workers)
-    pre = _lib.DecodePreludeArgs()
-    pre.q_proj, pre.k_proj, pre.v_proj = q_proj.data_ptr(), k_proj.data_ptr(), v_proj.data_ptr()
-    pre.inv_rms = inv_rms.data_ptr()
-    pre.q_norm_weight, pre.k_norm_weight = q_norm_weight.data_ptr(), k_norm_weight.data_ptr()
-    pre.rope_cos, pre.rope_sin = rope_cos.data_ptr(), rope_sin.data_ptr()
-    pre.max_position = rope_cos.shape[0]
-    pre.eps = float(eps)
-    return args, pre
 
 
 def check_errors(device: torch.device | None = None) -> None:
