@@ -235,7 +235,11 @@ Plan make_plan(const SimplerHipPaDecodeArgs *a, const KernelPair &k) {  // k: th
         p.tiles_per_worker = kMlaRowsPerGroup / 16 * p.groups;
         p.row_groups = 1;
         p.threads = 256;
-        p.main = k.main;
+        // At most 64 rows: the kernels whose four waves share the rows. us per
+        // step against the 128-row form: 32 sequences of 32 rows, 200-6000
+        // tokens 35.4 against 42.2; 16 of 16 rows, 1000-30000 68 against 105;
+        // 32 of 64 rows, 500-8000 59 against 72 (32-token blocks alike).
+        p.main = p.rows <= 32 ? k.main_multi : p.rows <= 64 ? k.main_pair : k.main;
         if (a->num_workers > 0) {
             p.workers = a->num_workers;
         } else {

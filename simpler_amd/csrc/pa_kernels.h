@@ -1814,6 +1814,15 @@ __device__ __forceinline__ i32x4_t buffer_rsrc(const void *base, uint32_t num_re
                      __builtin_amdgcn_readfirstlane((int)num_records), 0x00020000};
 }
 
+// LDS-only workgroup barrier: waits for this wave's LDS accesses, not for the
+// vector-memory loads in flight (__syncthreads would wait for the next
+// block's fill).
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+}
+
 template <int BS, int DK, int DV, typename OutT>
 __device__ __forceinline__ void run_mla_segment(const KernelParams &P, const int slice, const int rgrp, const int b,
                                                 const int kvh, const int nblk, const int blk_begin, const int blk_end,
@@ -2179,14 +2188,287 @@ __device__ __forceinline__ void run_mla_segment(const KernelParams &P, const int
     }
 }
 
+// MLA decode with at most 64 query rows (few heads per GPU): the four waves of
+// a workgroup share RT row tiles of 32 rows. In pa_mla_kernel, which gives
+// each wave its own 32 rows, one or two of them would do all the math of a
+// block, longer than its fill takes; here wave w runs QK for one (32-token
+// tile, row tile) pair, w mod NT RT, and PV for dims 128w .. 128w + 127 of
+// every row. Between them the waves exchange the block max of each row and
+// P^T (bf16, in the lane layout PV reads) through LDS, behind two barriers
+// that leave the next block's fill in flight. m, f and l are kept by every
+// wave. Per block of 64 tokens and wave: 36 + 16 RT MFMAs against 136, so the
+// block's 74 KB fill is what bounds it (32 sequences of 32 rows, 105 MB, main
+// kernel and merge: 42.2 -> 35.4 us; 313 MB over 16 sequences 105 -> 68).
+// Layouts, fill and numerics as run_mla_segment.
+template <int BS, int DK, int DV, typename OutT, int RT>
+__device__ __forceinline__ void run_mla_few_segment(const KernelParams &P, const int slice, const int b, const int kvh,
+                                                    const int nblk, const int blk_begin, const int blk_end,
+                                                    const int slot, char *const smem0, char *const smem1,
+                                                    float *const xmax, char *const xp) {
+    using L = MlaLayout<DK>;
+    constexpr int RB = L::kRowBytes, RC = L::kRowChunks;
+    constexpr int NI = BS * RC / 64, NII = (NI + 3) / 4;  // 1 KB direct-to-LDS loads per block, and per wave
+    constexpr int KS = DK / 16, NT = BS / 32, PS = BS / 16;
+    constexpr int NM = DV / 128;  // O^T tiles of 32 dims per wave
+    constexpr int PAIRS = NT * RT;
+    static_assert(BS % 32 == 0 && (BS * RC) % 64 == 0 && PAIRS <= 4 && DV % 128 == 0, "shapes");
+
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int h = lane >> 5, j = lane & 31;
+    const int tq = (wave % PAIRS) % NT, rq = (wave % PAIRS) / NT;  // this wave's QK tile
+    const int ctx = min(max(P.context_lens[b], 0), P.max_blocks * BS);
+
+    // ---- Q of row tile rq (B operand of QK): row j, dims 16kk + 8h .. ----
+    u32x4_t qv[KS];
+    int rowlen = 0;
+    {
+        const int r = 32 * rq + j;
+        const bool in = r < P.rows;
+        const int i = in ? r / P.group : 0, hh = in ? r - i * P.group : 0;
+        const uint16_t *qrow = P.q + ((int64_t)(b * P.q_len + i) * P.num_heads + kvh * P.group + hh) * DK + 8 * h;
+#pragma unroll
+        for (int kk = 0; kk < KS; ++kk) qv[kk] = in ? ld16(qrow + 16 * kk) : (u32x4_t){0u, 0u, 0u, 0u};
+        if (in) rowlen = P.causal ? ctx - (P.q_len - 1 - i) : ctx;
+    }
+    const int min_rowlen = P.causal ? ctx - (P.q_len - 1 - (32 * rq) / P.group) : ctx;
+
+    const __attribute__((address_space(4))) int32_t *bt_row =
+        (const __attribute__((address_space(4))) int32_t *)(P.block_table + (int64_t)b * P.max_blocks);
+
+    // ---- fill (see run_mla_segment) ----
+    const uint32_t tok_b = (uint32_t)(P.k_token_stride * 2);
+    const char *k_head = reinterpret_cast<const char *>(P.k) + (int64_t)kvh * P.k_head_stride * 2;
+    const int p0 = 64 * wave + lane;
+    const int t0 = p0 / RC, c0 = p0 - (p0 / RC) * RC;
+    constexpr int kStepChunks = 256 % RC, kStepRows = 256 / RC;
+    const uint32_t fill_base = (uint32_t)t0 * tok_b + 16u * (uint32_t)c0;
+    const uint32_t fill_step = (uint32_t)kStepRows * tok_b + 16u * kStepChunks;
+    const uint32_t fill_wrap = tok_b - 16u * RC;
+    constexpr uint32_t kDivRC = (65536u + RC - 1) / RC;
+    struct Fill {
+        i32x4_t rsrc;
+        uint32_t lds;
+    };
+    auto fill_of = [&](int blk, char *dst, bool &bad) -> Fill {
+        const int raw = blk >= 0 ? bt_row[blk] : 0;
+        bad = blk >= 0 && (unsigned)raw >= (unsigned)P.num_pool_blocks;
+        const int phys = bad ? 0 : raw;
+        const int vvalid = (bad || blk < 0) ? 0 : min(BS, ctx - blk * BS);
+        return {buffer_rsrc(k_head + (int64_t)phys * P.k_block_stride * 2, (uint32_t)vvalid * tok_b),
+                (uint32_t)__builtin_amdgcn_readfirstlane(lds_addr_of(dst) + 1024u * wave)};
+    };
+    auto fill_one = [&](const Fill &f, int ii) {
+        if (NI % 4 == 0 || 4 * ii + wave < NI) {
+            const uint32_t k = __umul24((uint32_t)c0 + kStepChunks * ii, kDivRC) >> 16;
+            const uint32_t off = (uint32_t)(__mul24((int)k, (int)fill_wrap) + (int)(fill_base + ii * fill_step));
+            lds_fill16(f.rsrc, off, f.lds + 4096u * ii);
+        }
+    };
+
+    f32x16_t acc[RT][NM];
+    float m_run[RT], f_run[RT], l_run[RT];
+#pragma unroll
+    for (int r = 0; r < RT; ++r) {
+#pragma unroll
+        for (int mt = 0; mt < NM; ++mt)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[r][mt][e] = 0.f;
+        m_run[r] = f_run[r] = kNegClamp;
+        l_run[r] = 0.f;
+    }
+    constexpr float kLog2e = 1.4426950408889634f;
+    const bf16x2_t ones2 = __builtin_bit_cast(bf16x2_t, 0x3f803f80u);
+    auto swap_halves = [](float x) {  // the value of lane l ^ 32
+        const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+        return (f32x2_t){__uint_as_float(r[0]), __uint_as_float(r[1])};
+    };
+    const uint32_t kofs = (32 * tq + j) * RB + 16 * h;
+    const int g = lane >> 4, pc = lane & 15;
+    const uint32_t vofs = (4 * h + (pc >> 2)) * RB + 32 * (g & 1) + 8 * (pc & 3) + 256 * wave;
+
+    constexpr unsigned kWaitAll = 0x0070u;  // vmcnt(0) lgkmcnt(0)
+    bool bad_cur = false, any_bad = false;
+    {
+        const Fill f0 = fill_of(blk_begin, smem0, bad_cur);
+#pragma unroll
+        for (int ii = 0; ii < NII; ++ii) fill_one(f0, ii);
+    }
+    for (int blk = blk_begin; blk < blk_end; ++blk) {
+        const bool even = ((blk - blk_begin) & 1) == 0;
+        const char *const kb = even ? smem0 : smem1;
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_waitcnt(kWaitAll);
+        __builtin_amdgcn_s_barrier();  // every wave's fill landed; the other buffer is free
+        __builtin_amdgcn_sched_barrier(0);
+        bool bad_next = false;
+        const Fill next = fill_of(blk + 1 < blk_end ? blk + 1 : -1, even ? smem1 : smem0, bad_next);
+        any_bad |= bad_cur;
+        const bool first = blk == blk_begin;
+
+        // ---- QK: S^T of the wave's tile, the next fill spread over it ----
+        f32x16_t s;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) s[e] = 0.f;
+        constexpr int KA = 4;  // k-steps the K reads run ahead
+        u32x4_t kf[KA];
+#pragma unroll
+        for (int kk = 0; kk < KA; ++kk) kf[kk] = lds_ld16(kb, kofs + 32 * kk);
+#pragma unroll
+        for (int kk = 0; kk < KS; ++kk) {
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int ii = 0; ii < NII; ++ii)
+                if (ii * KS / NII == kk) fill_one(next, ii);
+            s = mma_32x32x16(kf[kk % KA], qv[kk], s);
+            if (kk + KA < KS) kf[kk % KA] = lds_ld16(kb, kofs + 32 * (kk + KA));
+        }
+
+        // ---- mask, block max (as run_mla_segment) ----
+        float sc = P.scale;
+        if (!(sc > 0.f)) {
+            s *= sc;
+            sc = 1.f;
+        }
+        const int blk0 = blk * BS;
+        if (bad_cur || blk0 + BS > min_rowlen) {
+            const int rvalid = bad_cur ? 0 : rowlen - blk0;
+#pragma unroll
+            for (int e = 0; e < 16; ++e)
+                if (32 * tq + 8 * (e >> 2) + 4 * h + (e & 3) >= rvalid) s[e] = -INFINITY;
+        }
+        float mx = -INFINITY;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) mx = fmaxf(mx, s[e]);
+        {
+            const f32x2_t x = swap_halves(mx);
+            mx = fmaxf(x[0], x[1]);
+        }
+        float mrow[RT];
+        if constexpr (PAIRS > 1) {
+            if (h == 0) xmax[(rq * NT + tq) * 32 + j] = mx;  // (waves of the same pair write the same values)
+            lds_barrier();
+#pragma unroll
+            for (int r = 0; r < RT; ++r) {
+                mrow[r] = xmax[r * NT * 32 + j];
+#pragma unroll
+                for (int t = 1; t < NT; ++t) mrow[r] = fmaxf(mrow[r], xmax[(r * NT + t) * 32 + j]);
+            }
+        } else {
+            mrow[0] = mx;
+        }
+        // ---- online merge in the block frame, for every row ----
+        float cf[RT], mb2[RT];
+#pragma unroll
+        for (int r = 0; r < RT; ++r) {
+            const float mb = fmaxf(mrow[r] * sc, kNegClamp);
+            const float mnew = first ? mb : fmaxf(m_run[r], mb);
+            const bool use = first || (mb >= mnew - kFrameGap);
+            cf[r] = first ? 0.f : (use ? __expf(f_run[r] - mb) : 1.f);
+            mb2[r] = use ? mb * kLog2e : INFINITY;  // a skipped block gives p = 0
+            m_run[r] = mnew;
+            if (use) f_run[r] = mb;
+        }
+        // ---- p of the wave's tile, then everybody's P^T ----
+        const float sc2 = sc * kLog2e, mq = RT == 1 ? mb2[0] : (rq == 0 ? mb2[0] : mb2[RT - 1]);
+        u32x4_t own[2];
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                own[ks][i] = pack_bf16x2(__builtin_amdgcn_exp2f(__builtin_fmaf(s[8 * ks + 2 * i], sc2, -mq)),
+                                         __builtin_amdgcn_exp2f(__builtin_fmaf(s[8 * ks + 2 * i + 1], sc2, -mq)));
+        u32x4_t pk[RT][PS];
+        if constexpr (PAIRS > 1) {
+#pragma unroll
+            for (int ks = 0; ks < 2; ++ks) lds_st16(xp, ((rq * PS + 2 * tq + ks) * 64 + lane) * 16, own[ks]);
+            lds_barrier();
+#pragma unroll
+            for (int r = 0; r < RT; ++r)
+#pragma unroll
+                for (int ks = 0; ks < PS; ++ks) pk[r][ks] = lds_ld16(xp, ((r * PS + ks) * 64 + lane) * 16);
+        } else {
+            pk[0][0] = own[0];
+            pk[0][1] = own[1];
+        }
+#pragma unroll
+        for (int r = 0; r < RT; ++r) {
+            float lsum = 0.f;
+#pragma unroll
+            for (int ks = 0; ks < PS; ++ks)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const unsigned w = pk[r][ks][i];  // (a bit cast of the element itself would take element 0)
+                    lsum = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, w), ones2, lsum, false);
+                }
+            const f32x2_t x = swap_halves(lsum);  // the row's tokens of the other lane half
+            l_run[r] = l_run[r] * cf[r] + (x[0] + x[1]);
+#pragma unroll
+            for (int mt = 0; mt < NM; ++mt) acc[r][mt] *= cf[r];
+        }
+        // ---- A' = e^{f - m_blk} A + P V over the wave's dims ----
+#pragma unroll
+        for (int ks = 0; ks < PS; ++ks) {
+            i16x4_t vf[NM][2];
+#pragma unroll
+            for (int mt = 0; mt < NM; ++mt) {
+                vf[mt][0] = lds_ld_tr(kb, vofs + 64 * mt + 16 * ks * RB);
+                vf[mt][1] = lds_ld_tr(kb, vofs + 64 * mt + (16 * ks + 8) * RB);
+            }
+#pragma unroll
+            for (int mt = 0; mt < NM; ++mt) {
+                const u32x4_t va = __builtin_bit_cast(
+                    u32x4_t, __builtin_shufflevector(vf[mt][0], vf[mt][1], 0, 1, 2, 3, 4, 5, 6, 7));
+#pragma unroll
+                for (int r = 0; r < RT; ++r) acc[r][mt] = mma_32x32x16(va, pk[r][ks], acc[r][mt]);
+            }
+        }
+        bad_cur = bad_next;
+    }
+    __builtin_amdgcn_s_waitcnt(kWaitAll);  // the last zero fill is done before the next segment's
+    if (any_bad && threadIdx.x == 0) atomicOr(P.error_flag, kErrBadBlock);
+    __syncthreads();  // the buffers are refilled by the next segment
+
+    // ---- finish: lane (h, j) holds dims 128 wave + 32mt + 8a + 4h + e of row 32r + j ----
+#pragma unroll
+    for (int r = 0; r < RT; ++r) {
+        const int row = 32 * r + j;
+        if (row >= P.rows) continue;
+        const bool whole = blk_begin == 0 && blk_end == nblk;
+        const float inv = l_run[r] > 0.f ? 1.f / l_run[r] : 0.f;  // the frame factor cancels
+        const float osc = __expf(f_run[r] - m_run[r]);
+        const int64_t off = out_row_offset(P, b, kvh, row, DV) + 128 * wave + 4 * h;
+        const int64_t piece = ((int64_t)slice * P.tiles_per_worker + (row >> 4)) * 2 + slot;
+        float *dst = P.part_o + (piece * 16 + (row & 15)) * DV + 128 * wave + 4 * h;
+#pragma unroll
+        for (int mt = 0; mt < NM; ++mt)
+#pragma unroll
+            for (int a = 0; a < 4; ++a) {
+                const f32x4_t v = (f32x4_t){acc[r][mt][4 * a], acc[r][mt][4 * a + 1], acc[r][mt][4 * a + 2],
+                                            acc[r][mt][4 * a + 3]};
+                if (whole)
+                    OutStore<OutT>::store4(P.out, off + 32 * mt + 8 * a, v * inv);
+                else  // a piece of the tile per 16 rows: O relative to m, m and l
+                    *reinterpret_cast<f32x4_t *>(dst + 32 * mt + 8 * a) = v * osc;
+            }
+        if (!whole && wave == 0 && h == 0) {
+            P.part_ml[piece * 32 + (row & 15)] = m_run[r];
+            P.part_ml[piece * 32 + 16 + (row & 15)] = l_run[r] * osc;
+        }
+    }
+}
+
 // Worker workgroup = four waves = one row group (up to 128 query rows) of one
 // work slice. The work list holds (batch, kv head, KV block) entries; every
-// row group of a slice walks the same entries.
-template <int BS, int DK, int DV, typename OutT>
+// row group of a slice walks the same entries. RT > 0: at most 32 RT rows
+// (run_mla_few_segment).
+template <int BS, int DK, int DV, typename OutT, int RT = 0>
 __global__ void __launch_bounds__(256) pa_mla_kernel(const KernelParams P) {
     using L = MlaLayout<DK>;
     __shared__ __attribute__((aligned(16))) char smem0[BS * L::kRowBytes];
     __shared__ __attribute__((aligned(16))) char smem1[BS * L::kRowBytes];
+    __shared__ __attribute__((aligned(16))) char xp[RT ? RT * (BS / 16) * 1024 : 16];
+    __shared__ float xmax[RT ? RT * BS : 1];
     flag_bad_lengths(P);
     const int groups = (P.rows + kMlaRowsPerGroup - 1) / kMlaRowsPerGroup;
     int slice = 0, rgrp = 0;
@@ -2211,7 +2493,11 @@ __global__ void __launch_bounds__(256) pa_mla_kernel(const KernelParams P) {
     while (nb > 0) {
         const int blk0 = max(0, start - t0 - P.seg_cost), blk1 = min(nb, end - t0 - P.seg_cost);
         if (blk1 > blk0) {
-            run_mla_segment<BS, DK, DV, OutT>(P, slice, rgrp, b, kvh, nb, blk0, blk1, slot, smem0, smem1);
+            if constexpr (RT > 0)
+                run_mla_few_segment<BS, DK, DV, OutT, RT>(P, slice, b, kvh, nb, blk0, blk1, slot, smem0, smem1, xmax,
+                                                          xp);
+            else
+                run_mla_segment<BS, DK, DV, OutT>(P, slice, rgrp, b, kvh, nb, blk0, blk1, slot, smem0, smem1);
             slot = 1;
         }
         t0 += nb + P.seg_cost;
@@ -2239,10 +2525,10 @@ constexpr int kMlaDk = 576, kMlaDv = 512;
 
 struct KernelPair {
     KernelFn main;        // one wave per worker (MLA: the four-wave LDS kernel); null if unsupported
-    KernelFn main_multi;  // up to kMaxWavesPerWorker waves per worker
+    KernelFn main_multi;  // up to kMaxWavesPerWorker waves per worker (MLA: at most 32 query rows)
     bool mla;
     bool klds;  // stages K through LDS (full-row K reads); main_multi in dynamic LDS, BS x 256 B per wave
-    KernelFn main_pair = nullptr;  // one wave per worker running two row tiles (K through LDS), or null
+    KernelFn main_pair = nullptr;  // one wave per worker running two row tiles (K through LDS; MLA: 33 to 64 rows), or null
 };
 
 // Short-context decode (pa_kernels_direct.h): one workgroup of up to

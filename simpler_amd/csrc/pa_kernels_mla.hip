@@ -6,12 +6,22 @@
 namespace simpler_hip {
 namespace pa {
 
+namespace {
+
+template <int BS, typename OutT>
+KernelPair mla_set() {
+    return {pa_mla_kernel<BS, kMlaDk, kMlaDv, OutT>, pa_mla_kernel<BS, kMlaDk, kMlaDv, OutT, 1>, true, false,
+            pa_mla_kernel<BS, kMlaDk, kMlaDv, OutT, 2>};
+}
+
+}  // namespace
+
 KernelPair pick_mla(int bs, int out_dtype) {
     const bool f32 = out_dtype == SIMPLER_HIP_DT_FLOAT32, b16 = out_dtype == SIMPLER_HIP_DT_BFLOAT16;
-    if (bs == 32 && f32) return {pa_mla_kernel<32, kMlaDk, kMlaDv, float>, nullptr, true, false};
-    if (bs == 32 && b16) return {pa_mla_kernel<32, kMlaDk, kMlaDv, __bf16>, nullptr, true, false};
-    if (bs == 64 && f32) return {pa_mla_kernel<64, kMlaDk, kMlaDv, float>, nullptr, true, false};
-    if (bs == 64 && b16) return {pa_mla_kernel<64, kMlaDk, kMlaDv, __bf16>, nullptr, true, false};
+    if (bs == 32 && f32) return mla_set<32, float>();
+    if (bs == 32 && b16) return mla_set<32, __bf16>();
+    if (bs == 64 && f32) return mla_set<64, float>();
+    if (bs == 64 && b16) return mla_set<64, __bf16>();
     return KernelPair{};
 }
 
