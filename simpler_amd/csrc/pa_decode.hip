@@ -346,6 +346,25 @@ int direct_waves(const SimplerHipPaDecodeArgs *a, const Kernels &s, const Plan &
     return (int)waves;
 }
 
+// MLA: whether each tile runs whole, in a launch of one workgroup per (tile,
+// 128 rows), without the work lists and the merge. Short contexts only, as the
+// host knows the table's width and not the lengths: with few workgroups a tile
+// cut into blocks ends earlier. us per step against the work lists, 16 / 64 /
+// 128 rows, 64-token blocks:
+// - to 128 tokens always: one sequence 10.6 / 15.5 / 21.1 against 13.5 / 18.1 /
+//   23.0, 128 of them 11.7 / 17.6 / 23.9 against 19.8 / 27.9 / 35.6;
+// - to 256 from 32 workgroups: 32 of 128-256 tokens 14.5 / 20.3 / 28.9 against
+//   15.3 / 26.3 / 31.6 (8 of them 14.5 / 20.0 / 28.1 against 14.0 / 20.0 / 26.5);
+// - to 512 from 128 workgroups: 128 of 64-512 tokens 23.3 / 31.0 / 43.9 against
+//   26.7 / 38.8 / 52.4 (64 of 256-512 22.9 / 30.3 / 43.1 against 20.5 / 31.5 /
+//   41.7; 300 of 256-1024 73 / 87 / 120 against 69 / 88 / 121).
+bool mla_whole_tiles(const SimplerHipPaDecodeArgs *a, const Kernels &s, const Plan &p) {
+    if (!s.k.mla || a->num_workers > 0) return false;
+    const int64_t groups = (int64_t)a->batch * a->num_kv_heads * p.groups;
+    const int64_t tokens = (int64_t)a->max_blocks_per_seq * a->block_size;
+    return tokens <= (groups >= 128 ? 512 : groups >= 32 ? 256 : 128);
+}
+
 // Writes the error word into the host's mirror, after everything before it on
 // the stream.
 __global__ void mirror_kernel(const unsigned *flag, unsigned *mirror) {
@@ -512,10 +531,16 @@ int pa_decode_launch(const SimplerHipPaDecodeArgs *a, void *workspace, size_t wo
     P.v_new = (const uint16_t *)v_new;
 
     const int64_t tiles = (int64_t)a->batch * a->num_kv_heads * plan.row_tiles;
-    if (const int waves = append ? 0 : direct_waves(a, s, plan)) {
+    const int waves = append ? 0 : direct_waves(a, s, plan);
+    P.whole_tiles = mla_whole_tiles(a, s, plan);
+    if (waves || P.whole_tiles) {  // one launch; the mirror's, if any, follows
         if (phases & SIMPLER_HIP_PHASE_MAIN) {
-            hipLaunchKernelGGL(s.direct.fn, dim3((unsigned)tiles), dim3(64u * waves),
-                               (unsigned)(waves * s.direct.wave_lds), (hipStream_t)stream, P);
+            if (waves)
+                hipLaunchKernelGGL(s.direct.fn, dim3((unsigned)tiles), dim3(64u * waves),
+                                   (unsigned)(waves * s.direct.wave_lds), (hipStream_t)stream, P);
+            else
+                hipLaunchKernelGGL(plan.main, dim3((unsigned)(a->batch * a->num_kv_heads * plan.groups)),
+                                   dim3((unsigned)plan.threads), 0, (hipStream_t)stream, P);
             if (hipGetLastError() != hipSuccess) return SIMPLER_HIP_ERR_LAUNCH;
         }
         if (P.err_mirror) {

@@ -131,6 +131,7 @@ struct KernelParams {
     const uint16_t *k_new;
     const uint16_t *v_new;
     int32_t merge_units;  // merge kernel: 16-byte units of a tile per workgroup
+    int32_t whole_tiles;  // MLA: a workgroup per tile and row group, no work list, no merge
 };
 
 __device__ __forceinline__ u32x4_t ld16(const uint16_t *p) { return *reinterpret_cast<const u32x4_t *>(p); }
@@ -2458,6 +2459,16 @@ __device__ __forceinline__ void run_mla_few_segment(const KernelParams &P, const
     }
 }
 
+// An empty context of a whole-tile launch: zeros, as the merge kernel writes.
+template <int DV, typename OutT>
+__device__ __forceinline__ void mla_zero_rows(const KernelParams &P, const int b, const int kvh, const int rgrp) {
+    const int row0 = rgrp * kMlaRowsPerGroup;
+    const int units = min(kMlaRowsPerGroup, P.rows - row0) * (DV / 4);
+    for (int u = threadIdx.x; u < units; u += blockDim.x)
+        OutStore<OutT>::store4(P.out, out_row_offset(P, b, kvh, row0 + u / (DV / 4), DV) + 4 * (u % (DV / 4)),
+                               (f32x4_t){0.f, 0.f, 0.f, 0.f});
+}
+
 // Worker workgroup = four waves = one row group (up to 128 query rows) of one
 // work slice. The work list holds (batch, kv head, KV block) entries; every
 // row group of a slice walks the same entries. RT > 0: at most 32 RT rows
@@ -2472,10 +2483,21 @@ __global__ void __launch_bounds__(256) pa_mla_kernel(const KernelParams P) {
     flag_bad_lengths(P);
     const int groups = (P.rows + kMlaRowsPerGroup - 1) / kMlaRowsPerGroup;
     int slice = 0, rgrp = 0;
-    mla_worker(blockIdx.x, P.workers, groups, &slice, &rgrp);
     const int tpb = P.kv_heads;  // work-list tiles per batch
     int start = 0, end = 0, b = 0, prefix = 0, ctx0 = 0;
-    locate_slice(P, slice, &start, &end, &b, &prefix, &ctx0);  // identical in every wave
+    if (P.whole_tiles) {  // short contexts: this workgroup's tile, whole, as its only slice
+        const int tile = blockIdx.x / groups;
+        rgrp = blockIdx.x - tile * groups;
+        b = tile / tpb;
+        ctx0 = min(max(P.context_lens[b], 0), P.max_blocks * BS);
+        const int span = (ctx0 + BS - 1) / BS + P.seg_cost;
+        start = (tile - b * tpb) * span;
+        end = start + span;
+        if (ctx0 == 0) mla_zero_rows<DV, OutT>(P, b, tile - b * tpb, rgrp);
+    } else {
+        mla_worker(blockIdx.x, P.workers, groups, &slice, &rgrp);
+        locate_slice(P, slice, &start, &end, &b, &prefix, &ctx0);  // identical in every wave
+    }
     // wave-uniform values, kept in scalar registers
     start = __builtin_amdgcn_readfirstlane(start);
     end = __builtin_amdgcn_readfirstlane(end);

@@ -1,7 +1,7 @@
 """MLA decode with at most 64 query rows (the waves of a workgroup share the
 rows): one and two row tiles of 32, partly filled, both block sizes, causal
 rows, partial and whole contexts, scales of either sign, and the first row
-count of the 128-row form."""
+count of the 128-row form; and short contexts (a workgroup per whole tile)."""
 
 from __future__ import annotations
 
@@ -36,6 +36,48 @@ def test_few_rows(bs, heads, q_len, lens, workers, scale, device):
                                     scale=case.scale, causal=case.config.causal, num_workers=workers)
     assert_close(got.cpu().numpy(), oracle_numpy(case), what=f"mla h{heads} q{q_len} bs{bs}")
     pa.check_errors(device)
+
+
+@pytest.mark.parametrize("heads,kv_heads,q_len,bs,batch,width,longest", [
+    (16, 1, 1, 64, 1, 2, 128),       # the smallest launch
+    (16, 1, 2, 64, 3, 2, 128),
+    (65, 1, 2, 32, 5, 4, 128),       # two row groups, the second partly filled
+    (16, 1, 1, 64, 2, 3, 192),       # too long for two workgroups: work lists
+    (33, 1, 1, 64, 32, 4, 256),      # 32 workgroups
+    (4, 2, 4, 32, 16, 8, 256),       # two kv heads
+    (128, 1, 2, 64, 64, 8, 512),     # 128 workgroups
+    (16, 1, 1, 64, 129, 8, 512),
+])
+def test_whole_tiles(heads, kv_heads, q_len, bs, batch, width, longest, device):
+    """Against the oracle and the work lists (a forced worker count)."""
+    lens = [max(q_len, longest - 37 * i % longest) for i in range(batch)]
+    if batch > 2:
+        lens[1] = 0
+    lens[0] = longest
+    if q_len > 1:
+        lens = [max(n, q_len) for n in lens]
+    print(f"[case] h={heads} kvh={kv_heads} q={q_len} bs={bs} b={batch} w={width}", flush=True)
+    case = make_custom_case(batch=batch, num_heads=heads, kv_heads=kv_heads, head_dim=576, head_dim_v=512,
+                            block_size=bs, q_len=q_len, causal=q_len > 1, context_lens=lens, seed=1700 + heads,
+                            mla=True)
+    assert case.block_table.shape[1] == width
+    d = case.to(device)
+    outs = []
+    for workers in (0, 300):
+        out = torch.full((*d.query.shape[:-1], 512), float("nan"), device=device, dtype=torch.float32)
+        pa.paged_attention_decode(d.query, d.key_cache, d.value_cache, d.block_table, d.context_lens, out=out,
+                                  scale=case.scale, causal=case.config.causal, num_workers=workers)
+        outs.append(out)
+    assert_close(outs[0].cpu().numpy(), oracle_numpy(case), what=f"whole tiles h{heads} b{batch}")
+    # the same block frames, summed in another order
+    assert torch.allclose(outs[0], outs[1], rtol=1e-4, atol=1e-5)
+    pa.check_errors(device)
+    d.context_lens[0] = longest + 1  # past the table: clamped, and reported
+    pa.paged_attention_decode(d.query, d.key_cache, d.value_cache, d.block_table, d.context_lens, out=outs[1],
+                              scale=case.scale, causal=case.config.causal)
+    with pytest.raises(pa.PagedAttentionError):
+        pa.check_errors(device)
+    assert torch.equal(outs[0], outs[1])
 
 
 def test_bad_blocks_and_garbage_past_the_context(device):
