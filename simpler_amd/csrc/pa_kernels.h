@@ -1609,16 +1609,14 @@ pa_merge_kernel(const KernelParams P) {
     auto piece_ml = [&](int k, int row) { return ml_base + (k * step + (k == 0 ? slot0 : 0)) * 32 + row; };
 
     const int r0 = unit0 / UPR, nr = (unit0 + units - 1) / UPR - r0 + 1;  // its rows
-    const int np1 = np | 1;  // row stride of the LDS tables (odd: no bank conflicts)
-    if (nr * np1 > kMergeTable) {  // contexts cut finer than the default plans cut
+    if (nr * np > kMergeTable) {  // contexts cut finer than the default plans cut
         for (int u = tid; u < units; u += MT) {
             const int row = (unit0 + u) / UPR;
             float M = -INFINITY;
-#pragma unroll 1
             for (int k = 0; k < np; ++k) M = fmaxf(M, *piece_ml(k, row));
             float L = 0.f;
             f32x4_t o = (f32x4_t){0.f, 0.f, 0.f, 0.f};
-#pragma unroll 2
+#pragma unroll 4
             for (int k = 0; k < np; ++k) {
                 const float c = __expf(*piece_ml(k, row) - M);
                 L += c * piece_ml(k, row)[16];
@@ -1645,22 +1643,18 @@ pa_merge_kernel(const KernelParams P) {
     __shared__ float wgt[kMergeTable], lsum[kMergeTable];  // [row][piece]: m, then its weight; l
     __shared__ float row_inv[16];
     __shared__ f32x4_t part[UPT == 1 ? kMergeThreads : 1];
-    const int rsh = 32 - __clz(nr - 1);  // (0 for one row)
-    for (int e = tid; e < np << rsh; e += MT) {  // all (m, l) loads in flight at once
-        const int r = e & ((1 << rsh) - 1), k = e >> rsh;
-        if (r < nr) {
-            const float *ml = piece_ml(k, r0 + r);
-            wgt[r * np1 + k] = ml[0];
-            lsum[r * np1 + k] = ml[16];
-        }
+    for (int e = tid; e < nr * np; e += MT) {  // all (m, l) loads in flight at once
+        const int r = e / np;
+        const float *ml = piece_ml(e - r * np, r0 + r);
+        wgt[e] = ml[0];
+        lsum[e] = ml[16];
     }
     __syncthreads();
     const int lanes = np <= 16 ? 16 : 64;  // per row
     for (int r = tid / lanes; r < nr; r += MT / lanes) {
         const int l0 = tid & (lanes - 1);
-        float *const w = wgt + r * np1, *const ls = lsum + r * np1;
+        float *const w = wgt + r * np, *const ls = lsum + r * np;
         float M = -INFINITY;
-#pragma unroll 1
         for (int k = l0; k < np; k += lanes) M = fmaxf(M, w[k]);
         M = row16_combine(M, [](float x, float y) { return fmaxf(x, y); });
         if (lanes == 64) {
@@ -1668,7 +1662,6 @@ pa_merge_kernel(const KernelParams P) {
             M = fmaxf(M, __shfl_xor(M, 32, 64));
         }
         float L = 0.f;
-#pragma unroll 1
         for (int k = l0; k < np; k += lanes) {
             const float c = __expf(w[k] - M);
             w[k] = c;
@@ -1688,15 +1681,12 @@ pa_merge_kernel(const KernelParams P) {
         f32x4_t o = (f32x4_t){0.f, 0.f, 0.f, 0.f};
         if (u < units && g < G) {
             const int r = (unit0 + u) / UPR - r0;
-            const float *const w = wgt + r * np1;
+            const float *const w = wgt + r * np;
 #pragma unroll
             for (int i = 0; i < PRE; ++i)
                 if (g + i * G < np) o += w[g + i * G] * pre[n][i];
-            const float *src = o_base + (g + PRE * G) * step * (16 * DV) + 4 * (unit0 + u);  // past piece 0: slot 0
-            const int64_t stride = G * step * (16 * DV);
 #pragma unroll 4
-            for (int k = g + PRE * G; k < np; k += G, src += stride)
-                o += w[k] * *reinterpret_cast<const f32x4_t *>(src);
+            for (int k = g + PRE * G; k < np; k += G) o += w[k] * piece_unit(k, unit0 + u);
             o *= row_inv[r];
         }
         if (G > 1) {  // (UPT == 1)
