@@ -1539,6 +1539,20 @@ __device__ __forceinline__ float row16_combine(float x, F f) {
     return x;
 }
 
+// sum_k c_k l_k over lanes k < N of a row of 16, in the order of the lanes (a
+// fused multiply-add each), in every lane; L is lane k's own c_k l_k, and 0
+// past the last one. Lane k adds to the sum of the lane below, right after k
+// steps.
+template <int N>
+__device__ __forceinline__ float row16_ordered_sum(const float c, const float l, float L) {
+#pragma unroll
+    for (int i = 1; i < N; ++i)
+        L = __builtin_fmaf(
+            c, l, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(L), 0x111, 0xf, 0xf, true)));  // row_shr:1
+    return __int_as_float(
+        __builtin_amdgcn_update_dpp(0, __float_as_int(L), 0x150 + N - 1, 0xf, 0xf, true));  // row_newbcast:N-1
+}
+
 // O = sum_w e^{m_w - M} O_w / L over a tile's pieces w. The merge is bound by
 // memory latency (kernel arguments, lengths, pieces: three round trips), so
 // every piece load that can be is in flight at once. A tile's 16-byte units
@@ -1639,9 +1653,11 @@ pa_merge_kernel(const KernelParams P) {
                                                                : (f32x4_t){0.f, 0.f, 0.f, 0.f};
     }
 
-    // Weights e^{m_w - M} / L of the rows r0 .. r0 + nr - 1.
+    // Weights e^{m_w - M} / L of the rows r0 .. r0 + nr - 1. Up to 16 pieces, L
+    // is summed in their order, and O too where one thread takes them all, as
+    // the short-context kernel does: both give the same bits for the same
+    // pieces.
     __shared__ float wgt[kMergeTable], lsum[kMergeTable];  // [row][piece]: m, then its weight; l
-    __shared__ float row_inv[16];
     __shared__ f32x4_t part[UPT == 1 ? kMergeThreads : 1];
     for (int e = tid; e < nr * np; e += MT) {  // all (m, l) loads in flight at once
         const int r = e / np;
@@ -1650,29 +1666,41 @@ pa_merge_kernel(const KernelParams P) {
         lsum[e] = ml[16];
     }
     __syncthreads();
-    const int lanes = np <= 16 ? 16 : 64;  // per row
-    for (int r = tid / lanes; r < nr; r += MT / lanes) {
-        const int l0 = tid & (lanes - 1);
-        float *const w = wgt + r * np, *const ls = lsum + r * np;
-        float M = -INFINITY;
-        for (int k = l0; k < np; k += lanes) M = fmaxf(M, w[k]);
-        M = row16_combine(M, [](float x, float y) { return fmaxf(x, y); });
-        if (lanes == 64) {
+    if (np <= 16) {  // 16 lanes per row, a piece each
+        for (int r = tid >> 4; r < nr; r += MT >> 4) {
+            const int k = tid & 15;
+            const float m = k < np ? wgt[r * np + k] : -INFINITY, l = k < np ? lsum[r * np + k] : 0.f;
+            const float M = row16_combine(m, [](float x, float y) { return fmaxf(x, y); });
+            const float c = k < np ? __expf(m - M) : 0.f;
+            float L = c * l;
+            if (np <= 4)
+                L = row16_ordered_sum<4>(c, l, L);
+            else if (np <= 8)
+                L = row16_ordered_sum<8>(c, l, L);
+            else
+                L = row16_ordered_sum<16>(c, l, L);
+            if (k < np) wgt[r * np + k] = c * (L > 0.f ? 1.f / L : 0.f);
+        }
+    } else {  // a wave per row
+        for (int r = tid >> 6; r < nr; r += MT >> 6) {
+            float *const w = wgt + r * np, *const ls = lsum + r * np;
+            float M = -INFINITY;
+            for (int k = tid & 63; k < np; k += 64) M = fmaxf(M, w[k]);
+            M = row16_combine(M, [](float x, float y) { return fmaxf(x, y); });
             M = fmaxf(M, __shfl_xor(M, 16, 64));
             M = fmaxf(M, __shfl_xor(M, 32, 64));
-        }
-        float L = 0.f;
-        for (int k = l0; k < np; k += lanes) {
-            const float c = __expf(w[k] - M);
-            w[k] = c;
-            L += c * ls[k];
-        }
-        L = row16_combine(L, [](float x, float y) { return x + y; });
-        if (lanes == 64) {
+            float L = 0.f;
+            for (int k = tid & 63; k < np; k += 64) {
+                const float c = __expf(w[k] - M);
+                w[k] = c;
+                L += c * ls[k];
+            }
+            L = row16_combine(L, [](float x, float y) { return x + y; });
             L += __shfl_xor(L, 16, 64);
             L += __shfl_xor(L, 32, 64);
+            const float inv = L > 0.f ? 1.f / L : 0.f;
+            for (int k = tid & 63; k < np; k += 64) w[k] *= inv;
         }
-        if (l0 == 0) row_inv[r] = L > 0.f ? 1.f / L : 0.f;
     }
     __syncthreads();
 #pragma unroll
@@ -1687,7 +1715,6 @@ pa_merge_kernel(const KernelParams P) {
                 if (g + i * G < np) o += w[g + i * G] * pre[n][i];
 #pragma unroll 4
             for (int k = g + PRE * G; k < np; k += G) o += w[k] * piece_unit(k, unit0 + u);
-            o *= row_inv[r];
         }
         if (G > 1) {  // (UPT == 1)
             part[tid] = o;

@@ -66,23 +66,47 @@ __global__ void __launch_bounds__((64 * direct_max_waves<BS, D>())) pa_direct_ke
     const int pieces = (nb + per - 1) / per;
     if (pieces == 1) return;  // wave 0 stored the output
     __syncthreads();
-    // log-sum-exp merge of the waves' pieces
-    for (int u = threadIdx.x; u < units; u += blockDim.x) {
-        const int row = u / (D / 4), c = 4 * (u - row * (D / 4));
-        float M = -INFINITY;
-        for (int w = 0; w < pieces; ++w)
-            M = fmaxf(M, reinterpret_cast<const float *>(direct_lds + w * LW)[16 * D + row]);
-        float L = 0.f;
-        f32x4_t o = (f32x4_t){0.f, 0.f, 0.f, 0.f};
-        for (int w = 0; w < pieces; ++w) {
-            const float *const p = reinterpret_cast<const float *>(direct_lds + w * LW);
-            const float e = __expf(p[16 * D + row] - M);
-            L += e * p[16 * D + 16 + row];
-            o += e * *reinterpret_cast<const f32x4_t *>(p + row * D + c);
+    // log-sum-exp merge of the waves' pieces, in the arithmetic of the merge
+    // kernel: the weights are normalised first and the sums run in piece order,
+    // so a tile cut into the same pieces by the work lists has the same bits
+    auto merge = [&](auto most) {  // every LDS read of a unit in flight at once
+        constexpr int N = decltype(most)::value;
+        for (int u = threadIdx.x; u < units; u += blockDim.x) {
+            const int row = u / (D / 4), c = 4 * (u - row * (D / 4));
+            float m[N], l[N];
+            f32x4_t piece[N];
+#pragma unroll
+            for (int w = 0; w < N; ++w) {
+                const float *const p = reinterpret_cast<const float *>(direct_lds + min(w, pieces - 1) * LW);
+                m[w] = p[16 * D + row];
+                l[w] = p[16 * D + 16 + row];
+                piece[w] = *reinterpret_cast<const f32x4_t *>(p + row * D + c);
+            }
+            float M = m[0];
+#pragma unroll
+            for (int w = 1; w < N; ++w) M = fmaxf(M, m[w]);
+            float L = 0.f;
+#pragma unroll
+            for (int w = 0; w < N; ++w)
+                if (w < pieces) {
+                    m[w] = __expf(m[w] - M);
+                    L += m[w] * l[w];
+                }
+            const float inv = L > 0.f ? 1.f / L : 0.f;
+            f32x4_t o = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int w = 0; w < N; ++w)
+                if (w < pieces) o += (m[w] * inv) * piece[w];
+            OutStore<OutT>::store4(P.out, out_row_offset(P, b, kvh, rt * 16 + row, D) + c, o);
         }
-        const float inv = L > 0.f ? 1.f / L : 0.f;
-        OutStore<OutT>::store4(P.out, out_row_offset(P, b, kvh, rt * 16 + row, D) + c, o * inv);
-    }
+    };
+    constexpr int MAXW = direct_max_waves<BS, D>();
+    if (MAXW <= 4 || pieces <= 4)
+        merge(std::integral_constant<int, 4>{});
+    else if (MAXW <= 8 || pieces <= 8)
+        merge(std::integral_constant<int, MAXW < 8 ? MAXW : 8>{});
+    else
+        merge(std::integral_constant<int, MAXW>{});
 }
 
 template <int BS, int D, typename OutT, bool KV8, typename ET>

@@ -81,3 +81,34 @@ def test_errors_are_reported(device):
         pa.check_errors(device)
     assert e.value.rc == -6
     pa.check_errors(device)
+
+
+# (heads, kv heads, dim, block, lengths, cache format); one block per wave
+@pytest.mark.parametrize("hq,hkv,dim,bs,lens,kv", [
+    (16, 1, 128, 128, [512, 512], "bf16"),
+    (8, 2, 128, 128, [500, 129, 384], "bf16"),
+    (5, 1, 128, 16, [128, 3, 100], "fp16"),
+    (16, 4, 64, 32, [255, 64, 17], "fp16"),
+    (16, 2, 256, 64, [256, 70], "bf16"),
+    (4, 1, 256, 128, [256, 130], "bf16"),
+    (8, 1, 128, 64, [256, 200], "fp8"),
+])
+@pytest.mark.parametrize("out_dtype", [torch.float32, torch.bfloat16])
+def test_same_bits_as_the_work_lists(hq, hkv, dim, bs, lens, kv, out_dtype, device):
+    """A tile cut into the same pieces (a block each) by the work lists: the
+    pieces are the same and are merged in the same order, so the output is too."""
+    if kv == "fp16" and out_dtype == torch.bfloat16:
+        out_dtype = torch.float16
+    print(f"[case] {hq}/{hkv} d{dim} bs{bs} {lens} {kv} {out_dtype}", flush=True)
+    case = make_custom_case(batch=len(lens), num_heads=hq, kv_heads=hkv, head_dim=dim, block_size=bs,
+                            context_lens=lens, seed=1450 + dim + bs,
+                            dtype=torch.float16 if kv == "fp16" else torch.bfloat16)
+    if kv == "fp8":
+        case.key_cache, case.k_scale = quantize_kv_fp8(case.key_cache, pow2=False)
+        case.value_cache, case.v_scale = quantize_kv_fp8(case.value_cache, pow2=False)
+    a_worker_per_block = hkv * sum((n + bs - 1) // bs for n in lens)
+    d = case.to(device)
+    direct, lists = (pa.paged_attention_decode(d.query, d.key_cache, d.value_cache, d.block_table, d.context_lens,
+                                               scale=case.scale, out_dtype=out_dtype, num_workers=w,
+                                               k_scale=d.k_scale, v_scale=d.v_scale) for w in (0, a_worker_per_block))
+    assert torch.equal(direct, lists)
