@@ -243,7 +243,10 @@ Plan make_plan(const SimplerHipPaDecodeArgs *a, const KernelPair &k) {  // k: th
         if (a->num_workers > 0) {
             p.workers = a->num_workers;
         } else {
-            const int wgs = wave_slots(p.main, p.threads, kWorkersPerCu);
+            // One workgroup per CU: its two blocks fill half the LDS or more
+            // (a 32-token form whose registers let two run would double the
+            // partials, beyond the fixed scratch of the no-alloc entry).
+            const int wgs = wave_slots(p.main, p.threads, 1);
             p.workers = wgs / p.groups > 0 ? wgs / p.groups : 1;
         }
         p.grid = (int64_t)p.workers * p.groups;
@@ -686,10 +689,11 @@ namespace simpler_hip {
 namespace {
 
 // Every decode of the direct entry fits here at the default worker count on
-// MI355X (256 CUs): a GQA plan needs at most 2048 partial slots of 16 rows x
-// Dv fp32 (Dv 128: 16 MiB, Dv 256: 32 MiB), the MLA plan 4096 slots of 16 x 512
-// fp32 (256 slices x 8 row tiles x 2: 128 MiB), plus (m, l) pairs, the error
-// word and the zero page.
+// MI355X (256 CUs): a GQA plan has at most 12 waves per CU, 6144 partial slots
+// of 16 rows x Dv fp32, with head dims to 64 and fp8 caches (48 MiB at Dv 128),
+// and 2048 with 256 dims (32 MiB); the MLA plan 4096 slots of 16 x 512 fp32 (256
+// slices x 8 row tiles x 2: 128 MiB), plus (m, l) pairs, the error word and the
+// zero page.
 constexpr size_t kScratchBytes = (size_t)SIMPLER_HIP_PA_NOALLOC_SCRATCH_BYTES;
 static_assert(kScratchBytes % 256 == 0, "scratch size");
 

@@ -70,3 +70,29 @@ def test_noalloc_refuses_a_plan_beyond_its_scratch(device):
     assert _lib.lib().simpler_hip_pa_decode_noalloc(ctypes.byref(a), stream) == -4
     torch.cuda.synchronize(device)
     assert torch.count_nonzero(out).item() == 0  # nothing was launched
+
+
+@pytest.mark.parametrize("form", ["bf16", "fp16", "fp8", "mla"])
+def test_every_default_plan_fits_the_scratch(form, device):
+    """Workspace of the default plan over the supported head dims, block sizes and
+    row tiles per kv head, with token strides up to the largest zero page's."""
+    size = _lib.lib().simpler_hip_pa_decode_workspace_size
+    for dim in (576,) if form == "mla" else (128,) if form == "fp8" else (16, 32, 64, 128, 256):
+        for bs in (32, 64) if form == "mla" else (16, 32, 64, 128):
+            for rows in (1, 16, 17, 33, 49, 64, 65, 80, 128, 129, 256, 400):
+                for token in (dim, 16384):
+                    a = _lib.PaDecodeArgs()
+                    a.query, a.key_cache, a.block_table, a.context_lens, a.out = 0x1000, 0x2000, 0x4000, 0x5000, 0x6000
+                    a.value_cache = 0x2000 if form == "mla" else 0x3000
+                    a.k_block_stride = a.v_block_stride = bs * token
+                    a.k_token_stride = a.v_token_stride = token
+                    a.k_head_stride = a.v_head_stride = dim
+                    a.batch, a.q_len, a.num_heads, a.num_kv_heads = 32, 1, rows, 1
+                    a.head_dim_k, a.head_dim_v, a.block_size = dim, 512 if form == "mla" else dim, bs
+                    a.max_blocks_per_seq, a.num_blocks, a.out_dtype, a.scale = 1000, 32000, 0, 0.1
+                    a.kv_format = {"fp8": pa.KV_FP8_E4M3, "fp16": pa.KV_FP16}.get(form, pa.KV_BF16)
+                    a.k_scale, a.v_scale = 0x7000, 0x8000
+                    assert 0 < size(ctypes.byref(a)) <= SCRATCH_BYTES, (dim, bs, rows, token)
+                    if form == "mla":  # one workgroup per CU
+                        cus = torch.cuda.get_device_properties(device).multi_processor_count
+                        assert pa.plan(a) == cus // ((rows + 127) // 128)
