@@ -245,8 +245,11 @@ int simpler_hip_pa_decode_prelude(const SimplerHipPaDecodeArgs *args, const Simp
  * unsupported or invalid). */
 size_t simpler_hip_pa_decode_prelude_workspace_size(const SimplerHipPaDecodeArgs *args);
 
-/* Measurement helpers: name of the main kernel the args select, and the
- * number of worker wavefronts a launch uses. */
+/* Measurement helpers: name of the main kernel the args select, and how many
+ * workers simpler_hip_pa_decode runs them with: the slices the work lists are
+ * divided into (MLA: each run by ceil(rows / 128) workgroups), or, where short
+ * contexts run without work lists, the 16-row tiles (one workgroup each; MLA:
+ * the (sequence, kv head) pairs). */
 const char *simpler_hip_pa_decode_kernel_name(const SimplerHipPaDecodeArgs *args);
 int simpler_hip_pa_decode_plan(const SimplerHipPaDecodeArgs *args, int32_t *num_workers);
 

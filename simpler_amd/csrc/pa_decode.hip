@@ -368,6 +368,18 @@ bool mla_whole_tiles(const SimplerHipPaDecodeArgs *a, const Kernels &s, const Pl
     return tokens <= (groups >= 128 ? 512 : groups >= 32 ? 256 : 128);
 }
 
+// How a plain decode runs: one workgroup of `waves` waves per tile
+// (pa_direct_kernel), an MLA workgroup per whole tile and row group, or, with
+// neither, the work lists.
+struct Route {
+    int waves;
+    bool whole;
+};
+
+Route pick_route(const SimplerHipPaDecodeArgs *a, const Kernels &s, const Plan &p) {
+    return {direct_waves(a, s, p), mla_whole_tiles(a, s, p)};
+}
+
 // Writes the error word into the host's mirror, after everything before it on
 // the stream.
 __global__ void mirror_kernel(const unsigned *flag, unsigned *mirror) {
@@ -457,7 +469,12 @@ extern "C" int simpler_hip_pa_decode_plan(const SimplerHipPaDecodeArgs *args, in
     if (rc != SIMPLER_HIP_OK) return rc;
     const Kernels s = pick_kernel(args);
     if (!s.k.main) return SIMPLER_HIP_ERR_UNSUPPORTED;
-    if (num_workers) *num_workers = make_plan(args, s.k).workers;
+    const Plan plan = make_plan(args, s.k);
+    const Route route = pick_route(args, s, plan);
+    if (num_workers)
+        *num_workers = route.waves   ? args->batch * args->num_kv_heads * plan.row_tiles
+                       : route.whole ? args->batch * args->num_kv_heads
+                                     : plan.workers;
     return SIMPLER_HIP_OK;
 }
 
@@ -465,7 +482,8 @@ extern "C" const char *simpler_hip_pa_decode_kernel_name(const SimplerHipPaDecod
     if (validate(args) != SIMPLER_HIP_OK) return "";
     const Kernels s = pick_kernel(args);
     if (!s.k.main) return "";
-    return s.k.mla ? "pa_mla_kernel" : "pa_decode_kernel";
+    if (s.k.mla) return "pa_mla_kernel";
+    return pick_route(args, s, make_plan(args, s.k)).waves ? "pa_direct_kernel" : "pa_decode_kernel";
 }
 
 extern "C" int simpler_hip_pa_decode(const SimplerHipPaDecodeArgs *a, void *workspace, size_t workspace_bytes,
@@ -534,13 +552,13 @@ int pa_decode_launch(const SimplerHipPaDecodeArgs *a, void *workspace, size_t wo
     P.v_new = (const uint16_t *)v_new;
 
     const int64_t tiles = (int64_t)a->batch * a->num_kv_heads * plan.row_tiles;
-    const int waves = append ? 0 : direct_waves(a, s, plan);
-    P.whole_tiles = mla_whole_tiles(a, s, plan);
-    if (waves || P.whole_tiles) {  // one launch; the mirror's, if any, follows
+    const Route route = append ? Route{} : pick_route(a, s, plan);
+    P.whole_tiles = route.whole;
+    if (route.waves || route.whole) {  // one launch; the mirror's, if any, follows
         if (phases & SIMPLER_HIP_PHASE_MAIN) {
-            if (waves)
-                hipLaunchKernelGGL(s.direct.fn, dim3((unsigned)tiles), dim3(64u * waves),
-                                   (unsigned)(waves * s.direct.wave_lds), (hipStream_t)stream, P);
+            if (route.waves)
+                hipLaunchKernelGGL(s.direct.fn, dim3((unsigned)tiles), dim3(64u * route.waves),
+                                   (unsigned)(route.waves * s.direct.wave_lds), (hipStream_t)stream, P);
             else
                 hipLaunchKernelGGL(plan.main, dim3((unsigned)(a->batch * a->num_kv_heads * plan.groups)),
                                    dim3((unsigned)plan.threads), 0, (hipStream_t)stream, P);
@@ -600,7 +618,7 @@ extern "C" int simpler_hip_pa_decode_append(const SimplerHipPaDecodeArgs *a, con
         const Kernels s = pick_kernel(a);
         if (s.k.main) {
             const Plan plan = make_plan(a, s.k);
-            if (plan.tiles_per_worker > 1 || s.k.mla || direct_waves(a, s, plan)) {
+            if (plan.tiles_per_worker > 1 || s.k.mla || pick_route(a, s, plan).waves) {
                 if (!workspace || workspace_bytes < plan.total || ((uintptr_t)workspace & 255))
                     return SIMPLER_HIP_ERR_WORKSPACE;
                 if (a->batch == 0) return SIMPLER_HIP_OK;

@@ -562,10 +562,11 @@ def check_errors(device: torch.device | None = None) -> None:
 
 
 def plan(args: _lib.PaDecodeArgs) -> int:
-    """Number of workers (work-list slices) a launch with ``args`` uses on the current device.
+    """Number of workers a launch with ``args`` uses on the current device.
 
-    A worker is one workgroup for the decode kernel and one slice run by
-    ceil(rows / 128) sibling workgroups for the MLA kernel.
+    A worker is a work-list slice (one workgroup for the decode kernel,
+    ceil(rows / 128) sibling workgroups for the MLA kernel) or, where short
+    contexts run without work lists, a whole tile.
     """
     n = ctypes.c_int32()
     rc = _lib.lib().simpler_hip_pa_decode_plan(ctypes.byref(args), ctypes.byref(n))

@@ -1,0 +1,88 @@
+"""Which way a decode runs, as the kernel name and the plan report it: work
+lists, or one workgroup per tile for short contexts (GQA: pa_direct_kernel; MLA:
+whole tiles), on both sides of the rules that decide."""
+
+from __future__ import annotations
+
+import pytest
+
+from simpler_amd import paged_attention as pa
+from tests.test_abi import _args, _mla_args
+
+# (heads, kv heads, dim, block size, batch, q_len, table width): the shapes of
+# test_direct_gpu.py, and whether they are short enough
+GQA = [
+    (4, 1, 16, 16, 6, 1, 16, True),
+    (16, 2, 64, 16, 3, 1, 32, True),
+    (8, 8, 128, 128, 4, 1, 4, True),
+    (10, 2, 128, 64, 2, 1, 4, True),
+    (8, 1, 128, 32, 3, 1, 8, True),
+    (4, 2, 256, 64, 2, 1, 4, True),
+    (4, 2, 256, 128, 2, 1, 1, True),
+    (40, 2, 128, 16, 2, 1, 8, True),
+    (32, 4, 64, 32, 3, 8, 4, True),
+    (32, 32, 64, 64, 5, 1, 16, True),
+    (16, 1, 128, 128, 2, 1, 5, False),  # two 64 KB blocks for a wave
+    (32, 8, 128, 128, 32, 1, 64, False),
+]
+
+
+def gqa(hq, hkv, d, bs, batch, q_len, width, **kw):
+    token = hkv * d
+    return _args(num_heads=hq, num_kv_heads=hkv, head_dim_k=d, head_dim_v=d, block_size=bs, batch=batch, q_len=q_len,
+                 causal=int(q_len > 1), max_blocks_per_seq=width, k_block_stride=bs * token, v_block_stride=bs * token,
+                 k_token_stride=token, v_token_stride=token, k_head_stride=d, v_head_stride=d, **kw)
+
+
+def check_gqa(hq, hkv, d, bs, batch, q_len, width, short, **kw):
+    a = gqa(hq, hkv, d, bs, batch, q_len, width, **kw)
+    assert pa.kernel_name(a) == ("pa_direct_kernel" if short else "pa_decode_kernel")
+    if short:  # a workgroup per tile
+        assert pa.plan(a) == batch * hkv * ((hq // hkv * q_len + 15) // 16)
+    a.num_workers = 9  # a forced count keeps the work lists
+    assert pa.kernel_name(a) == "pa_decode_kernel" and pa.plan(a) == 9
+
+
+# (heads, kv heads, batch, q_len, block size, width, whole tiles)
+MLA = [
+    (16, 1, 1, 1, 64, 2, True),
+    (16, 1, 2, 1, 64, 3, False),
+    (65, 1, 5, 2, 32, 4, True),
+    (33, 1, 32, 1, 64, 4, True),
+    (33, 1, 31, 1, 64, 4, False),
+    (4, 2, 16, 4, 32, 4, True),
+    (128, 1, 64, 2, 64, 8, True),
+    (128, 1, 63, 2, 64, 8, False),
+    (16, 1, 129, 1, 64, 8, True),
+    (16, 1, 129, 1, 64, 9, False),
+]
+
+
+def check_mla(heads, hkv, batch, q_len, bs, width, whole):
+    a = _mla_args(num_heads=heads, num_kv_heads=hkv, batch=batch, q_len=q_len, causal=int(q_len > 1), block_size=bs,
+                  max_blocks_per_seq=width)
+    assert pa.kernel_name(a) == "pa_mla_kernel"
+    groups = (heads // hkv * q_len + 127) // 128
+    assert pa.plan(a) == (batch * hkv if whole else 256 // groups)
+    a.num_workers = 9
+    assert pa.plan(a) == 9
+
+
+@pytest.mark.parametrize("row", GQA)
+@pytest.mark.parametrize("kv_format", [pa.KV_BF16, pa.KV_FP16])
+def test_gqa(row, kv_format):
+    check_gqa(*row, kv_format=kv_format, out_dtype=0)
+
+
+@pytest.mark.parametrize("row", MLA)
+def test_mla(row):
+    check_mla(*row)
+
+
+@pytest.mark.gpu
+def test_on_the_device(device):
+    """The same with the device's own CU and occupancy figures."""
+    for row in GQA:
+        check_gqa(*row)
+    for row in MLA:
+        check_mla(*row)
