@@ -10,6 +10,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <atomic>
 #include <mutex>
 #include <vector>
 
@@ -29,7 +30,6 @@ using namespace pa;
 constexpr int kZeroOffset = 128;  // workspace bytes [128, 256) are never written after init
 constexpr int kMaxAppendTokens = 16;  // fused append: new tokens per sequence (one per residue mod 16)
 constexpr size_t kMaxZeroPageBytes = 1 << 20;  // larger token strides read the padding tiles as they are
-constexpr int64_t kDirectManyTiles = 128, kDirectTileBytes = 512 << 10, kDirectWaveBytes = 48 << 10;  // direct_waves
 constexpr int kMlaSegTokens = 256;  // MLA: work charged for each sequence a slice starts, in tokens
 
 struct Plan {
@@ -137,10 +137,24 @@ int current_device() {
     return hipGetDevice(&dev) == hipSuccess ? dev : -1;
 }
 
+// Compute units of the current device; without one an MI355X is assumed.
+int cu_count() {
+    constexpr int kDevices = 64;
+    static std::atomic<int> known[kDevices];
+    const int dev = current_device();
+    if (dev < 0) return 256;
+    int n = dev < kDevices ? known[dev].load(std::memory_order_relaxed) : 0;
+    if (n > 0) return n;
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) {
+        (void)hipGetLastError();
+        return 256;
+    }
+    if (dev < kDevices) known[dev].store(n, std::memory_order_relaxed);
+    return n;
+}
+
 // Default worker count: compute units x the requested workgroups per CU
 // (workers_per_cu), capped by what the kernel's register footprint allows.
-// Without a device (host-only builds and tests) an MI355X is assumed:
-// 256 CUs.
 int wave_slots(KernelFn fn, int threads, int want_per_cu, size_t lds = 0) {
     struct Entry {
         KernelFn fn;
@@ -158,13 +172,11 @@ int wave_slots(KernelFn fn, int threads, int want_per_cu, size_t lds = 0) {
         if (e.fn == fn && e.device == dev && e.threads == threads && e.want == want_per_cu && e.lds == lds)
             return e.slots;
     int per_cu = want_per_cu;
-    int cus = 256;
+    const int cus = cu_count();
     // Without a device: the kernels use the whole register file of a SIMD
     // (one wave per SIMD, four SIMDs per CU), the MLA kernel most of the LDS.
     if (dev < 0) per_cu = std::max(1, std::min(per_cu, 256 / threads));
     if (dev >= 0) {
-        int v = 0;
-        if (hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && v > 0) cus = v;
         int n = 0;
         if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, reinterpret_cast<const void *>(fn),
                                                          threads, lds) == hipSuccess &&
@@ -314,38 +326,49 @@ Plan make_plan(const SimplerHipPaDecodeArgs *a, const KernelPair &k) {  // k: th
 // where the work lists run: the caller forced a worker count, or a context may
 // be long (the host knows the table's width, not the lengths). One workgroup
 // per tile saves the merge launch and the work scan, but does not balance
-// lengths, so it is taken where the longest possible tile is short:
-// - with 128 tiles or more, up to 512 KB of K and V per tile (1024 tokens of
-//   128 dims), for kernels that keep few bytes in flight (head dims to 64, fp8
-//   caches) up to 256 KB. us per step against the work lists, 8 kv heads, D =
-//   128, 128-token blocks: 32 sequences of 100-500 tokens 12.0 against 17.2,
-//   of 200-1000 19.1 against 22.7; 130 of 512 54.0 against 57.4; 256 of
-//   200-1000 113 against 125; 256 of 16-40 21.6 against 30.5. At twice the
-//   limit, 130 of 100-2048, 118 against 110. Every row tile of a kv head reads
-//   K and V again, so its tiles together stay within 768 KB (32 x 4 kv heads of
-//   64 rows, 100-500 tokens 20.7 against 23.5, 200-1000 34.4 against 27.8).
-// - with fewer tiles, where each wave takes one block at most, or 48 KB:
-//   2 sequences of 512 tokens and 1 kv head 7.9 against 10.6, of 16-40 tokens
-//   in 16-token blocks 5.0 against 8.3; at two 64 KB blocks per wave 16.2
-//   against 13.5.
+// lengths and has fewer waves for a tile, so it is taken where the longest
+// possible tile is short. us per step, this form / work lists, all sequences
+// as long as the table is wide or 10-30% to 100% of it:
+// - From 32 tiles: up to 384 KB of K and V per tile (16 to 100 sequences of 8
+//   kv heads, 128 dims, 0.55 to 0.92 of the lists' time; at 512 KB, 40 of 1024
+//   tokens 37.8 / 36.6, 100 of 102-1024 50.2 / 48.4). 256 KB with head dims to
+//   64 and fp8 caches (0.97 at most; 4 x 8 of 200-2000 tokens, 64 dims, 17.8 /
+//   15.4) and with 256 dims, there 384 KB from 128 tiles (0.96 at most) unless
+//   blocks exceed the registers (200 x 4, 51-512 tokens in 128-token blocks,
+//   512 KB, 72.8 / 65.1).
+// - Fewer tiles, whose chains the lists cut finer: 192 KB with head dims to 64
+//   and fp8 caches (0.97 at most; one sequence of 64 dims in 16-token blocks
+//   10.2 / 9.9 at 256 KB, 16.1 / 10.3 at 512), else 256 KB (128 dims 0.84 at
+//   most; 9.8 / 9.6 at 384), with 256 dims one block per wave (1.005 at most;
+//   with two 12.2 / 9.4).
+// - To 128 tiles one block per wave or 48 KB (two 64 KB blocks 16.2 / 13.5).
+// - Every row tile of a kv head reads K and V again: with several of them up to
+//   64 KB per tile (0.93 at most, to 8192 tiles) or 48 MB in all (0.97 at most;
+//   128 x 8 kv heads, 64 rows of 64 dims, 1000 tokens in 32-token blocks, 1 GB,
+//   174 / 127; 15 x 8 of 380 tokens, 64 rows of 128 dims, 90 MB, 23.5 / 20.9).
+//   Above 64 dims, 768 KB over the row tiles of a kv head at most.
 // Waves per tile: enough for workers_per_cu waves on every CU, at least four.
 int direct_waves(const SimplerHipPaDecodeArgs *a, const Kernels &s, const Plan &p) {
     if (!s.direct.fn || a->num_workers > 0) return 0;
-    const bool fp8 = a->kv_format == SIMPLER_HIP_KV_FP8_E4M3;
-    const int64_t blocks = a->max_blocks_per_seq;
-    const int64_t block_bytes = (int64_t)a->block_size * 2 * a->head_dim_k * (fp8 ? 1 : 2);
+    const int bs = a->block_size, d = a->head_dim_k;
+    const bool fp8 = a->kv_format == SIMPLER_HIP_KV_FP8_E4M3, narrow = fp8 || d <= 64;
+    const int64_t blocks = a->max_blocks_per_seq, block = (int64_t)bs * 2 * d * (fp8 ? 1 : 2);
+    const int64_t tile = blocks * block;
     const int64_t tiles = std::max<int64_t>((int64_t)a->batch * a->num_kv_heads * p.row_tiles, 1);
-    if (blocks * block_bytes > kDirectTileBytes) return 0;
+    constexpr int64_t KB = 1 << 10;
+    if (!narrow && p.row_tiles > 1 && tile * p.row_tiles > 768 * KB) return 0;
     Plan one = p;
     one.tiles_per_worker = 1;
-    const int64_t want = 256 * (int64_t)std::max(kWorkersPerSimdCu, workers_per_cu(a, s.k, one, false));
+    const int64_t want = (int64_t)cu_count() * std::max(kWorkersPerSimdCu, workers_per_cu(a, s.k, one, false));
     const int64_t waves = std::min<int64_t>({(want + tiles - 1) / tiles, s.direct.max_waves, blocks});
     const int64_t per_wave = (blocks + waves - 1) / waves;
-    const bool narrow = fp8 || a->head_dim_k <= 64;
-    if (!narrow && p.row_tiles > 1 && blocks * block_bytes * p.row_tiles > kDirectTileBytes * 3 / 2) return 0;
-    if (tiles >= kDirectManyTiles ? narrow && blocks * block_bytes > kDirectTileBytes / 2
-                                  : per_wave > 1 && per_wave * block_bytes > kDirectWaveBytes)
-        return 0;
+    if (tiles < 128 && per_wave > 1 && per_wave * block > 48 * KB) return 0;
+    if (tiles < 32 && per_wave > 1 && d > 128) return 0;
+    const int64_t most = narrow    ? (tiles < 32 ? 192 : 256)
+                         : d > 128 ? (tiles < 128 || bs * d > 16384 ? 256 : 384)
+                                   : (tiles < 32 ? 256 : 384);
+    if (tile > most * KB) return 0;
+    if (p.row_tiles > 1 && tile > 64 * KB && tiles * tile > 48 * KB * KB) return 0;
     return (int)waves;
 }
 

@@ -24,6 +24,44 @@ GQA = [
     (32, 32, 64, 64, 5, 1, 16, True),
     (16, 1, 128, 128, 2, 1, 5, False),  # two 64 KB blocks for a wave
     (32, 8, 128, 128, 32, 1, 64, False),
+    # below 32 tiles: bytes per tile
+    (4, 1, 64, 16, 1, 1, 48, True),     # 192 KB, three blocks for a wave
+    (4, 1, 64, 16, 1, 1, 49, False),
+    (4, 1, 64, 64, 31, 1, 12, True),
+    (4, 1, 64, 64, 31, 1, 13, False),
+    (4, 1, 128, 16, 31, 1, 32, True),   # 256 KB
+    (4, 1, 128, 16, 31, 1, 33, False),
+    (16, 4, 256, 16, 4, 1, 8, True),    # one block for a wave
+    (16, 4, 256, 16, 4, 1, 9, False),
+    (4, 1, 256, 128, 1, 1, 2, True),
+    (4, 1, 256, 128, 1, 1, 3, False),
+    # from 32 tiles
+    (4, 1, 64, 64, 32, 1, 16, True),    # 256 KB
+    (4, 1, 64, 64, 32, 1, 17, False),
+    (4, 1, 128, 16, 32, 1, 48, True),   # 384 KB
+    (4, 1, 128, 16, 32, 1, 49, False),
+    (32, 8, 128, 64, 8, 1, 4, True),    # one block for a wave, or 48 KB
+    (32, 8, 128, 64, 8, 1, 5, False),
+    (16, 4, 256, 16, 8, 1, 16, True),
+    (16, 4, 256, 16, 8, 1, 17, False),
+    # from 128 tiles
+    (32, 8, 128, 128, 16, 1, 6, True),  # 384 KB
+    (32, 8, 128, 128, 16, 1, 7, False),
+    (32, 8, 64, 16, 16, 1, 64, True),   # 256 KB
+    (32, 8, 64, 16, 16, 1, 65, False),
+    (32, 8, 256, 64, 16, 1, 6, True),
+    (32, 8, 256, 64, 16, 1, 7, False),
+    (32, 8, 256, 128, 16, 1, 2, True),  # blocks larger than the registers
+    (32, 8, 256, 128, 16, 1, 3, False),
+    # several row tiles: 64 KB per tile or 48 MB over all of them
+    (128, 8, 64, 32, 32, 4, 8, True),
+    (128, 8, 64, 32, 32, 4, 9, False),
+    (32, 2, 64, 32, 16, 4, 32, True),
+    (128, 8, 64, 128, 24, 4, 2, True),
+    (128, 8, 64, 128, 24, 4, 3, False),
+    (128, 8, 64, 128, 16, 4, 3, True),
+    (16, 1, 128, 16, 1, 4, 24, True),   # 768 KB over four row tiles
+    (16, 1, 128, 16, 1, 4, 25, False),
 ]
 
 
@@ -72,6 +110,15 @@ def check_mla(heads, hkv, batch, q_len, bs, width, whole):
 @pytest.mark.parametrize("kv_format", [pa.KV_BF16, pa.KV_FP16])
 def test_gqa(row, kv_format):
     check_gqa(*row, kv_format=kv_format, out_dtype=0)
+
+
+@pytest.mark.parametrize("row", [
+    (8, 1, 128, 16, 1, 1, 48, True), (8, 1, 128, 16, 1, 1, 49, False),   # few tiles: 192 KB
+    (64, 8, 128, 32, 16, 1, 32, True), (64, 8, 128, 32, 16, 1, 33, False),  # many: 256 KB
+    (128, 8, 128, 64, 128, 8, 4, True), (128, 8, 128, 64, 128, 8, 5, False),  # eight row tiles: 64 KB
+])
+def test_fp8(row):
+    check_gqa(*row, kv_format=pa.KV_FP8_E4M3, out_dtype=0, k_scale=0x7000, v_scale=0x8000)
 
 
 @pytest.mark.parametrize("row", MLA)
