@@ -384,11 +384,17 @@ int direct_waves(const SimplerHipPaDecodeArgs *a, const Kernels &s, const Plan &
 // - to 512 from 128 workgroups: 128 of 64-512 tokens 23.3 / 31.0 / 43.9 against
 //   26.7 / 38.8 / 52.4 (64 of 256-512 22.9 / 30.3 / 43.1 against 20.5 / 31.5 /
 //   41.7; 300 of 256-1024 73 / 87 / 120 against 69 / 88 / 121).
+// 32-token blocks are twice the steps: a quarter less where the workgroups are
+// fewest, below 8 (one sequence of 128 tokens, 96 rows 20.4 against 19.2; of 96
+// 0.95 of the lists' time at most) and from 32 to 63 (32 of 51-256 tokens, 16
+// rows 16.7 against 15.8; 0.93 at most to 192, and to 256 from 64 workgroups).
 bool mla_whole_tiles(const SimplerHipPaDecodeArgs *a, const Kernels &s, const Plan &p) {
     if (!s.k.mla || a->num_workers > 0) return false;
     const int64_t groups = (int64_t)a->batch * a->num_kv_heads * p.groups;
     const int64_t tokens = (int64_t)a->max_blocks_per_seq * a->block_size;
-    return tokens <= (groups >= 128 ? 512 : groups >= 32 ? 256 : 128);
+    int64_t most = groups >= 128 ? 512 : groups >= 32 ? 256 : 128;
+    if (a->block_size == 32 && (groups < 8 || (groups >= 32 && groups < 64))) most -= most / 4;
+    return tokens <= most;
 }
 
 // How a plain decode runs: one workgroup of `waves` waves per tile

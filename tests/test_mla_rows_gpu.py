@@ -44,7 +44,8 @@ def test_few_rows(bs, heads, q_len, lens, workers, scale, device):
     (65, 1, 2, 32, 5, 4, 128),       # two row groups, the second partly filled
     (16, 1, 1, 64, 2, 3, 192),       # too long for two workgroups: work lists
     (33, 1, 1, 64, 32, 4, 256),      # 32 workgroups
-    (4, 2, 4, 32, 16, 8, 256),       # two kv heads
+    (4, 2, 4, 32, 16, 6, 192),       # two kv heads
+    (4, 2, 4, 32, 16, 8, 256),       # too long for 32 workgroups with 32-token blocks: work lists
     (128, 1, 2, 64, 64, 8, 512),     # 128 workgroups
     (16, 1, 1, 64, 129, 8, 512),
 ])

@@ -93,6 +93,14 @@ MLA = [
     (128, 1, 63, 2, 64, 8, False),
     (16, 1, 129, 1, 64, 8, True),
     (16, 1, 129, 1, 64, 9, False),
+    # 32-token blocks with the fewest workgroups of each range
+    (96, 1, 7, 1, 32, 3, True),
+    (96, 1, 7, 1, 32, 4, False),
+    (96, 1, 8, 1, 32, 4, True),
+    (16, 1, 32, 1, 32, 6, True),
+    (16, 1, 32, 1, 32, 7, False),
+    (16, 1, 63, 1, 32, 7, False),
+    (16, 1, 64, 1, 32, 8, True),
 ]
 
 
