@@ -202,8 +202,10 @@ int wave_slots(KernelFn fn, int threads, int want_per_cu, size_t lds = 0) {
 //   tokens, 8 kv heads of 64 dims, at 2 / 4 / 6 / 8 per CU: 16-token blocks
 //   104.4 / 60.1 / 43.5 / 36.2; 32: 71.8 / 42.3 / 34.5 / 36.3; 64: 55.9 / 37.2
 //   / 37.8 / 37.1; 128: 58.6 / 37.8 / 49.5 / 43.3. fp8 (32 sequences to 8192)
-//   at 3 / 4 / 8: 101.4 / 79.6 / 54.2; 66.8 / 54.9 / 57.8; 54.2 / 57.1 / 58.2;
-//   59.1 / 56.5 / 57.6.
+//   at 3 / 4 / 8: 101.4 / 79.6 / 54.2; 66.8 / 54.9 / 57.8; 54.2 / 57.1 / 58.2.
+//   128-token fp8 blocks: three; four was up to 4% faster with some lengths and
+//   up to 3% slower with others (steps of 32 sequences of 1024-8192 tokens at
+//   3 / 4, three draws: 62.7 / 60.5, 63.0 / 64.1, 58.3 / 59.4).
 // - 256-dim heads: two (four and more measured 2-8% slower), but four where a
 //   block exceeds the registers and runs unpipelined (151.6 against 170.7).
 // - Sibling waves (several row tiles per worker): the same by waves, since
@@ -229,7 +231,7 @@ int workers_per_cu(const SimplerHipPaDecodeArgs *a, const KernelPair &k, const P
     }
     if (k.klds) return kWorkersPerSimdCu;
     if (nominal) return fp8 ? kWorkersThreePerCu : kWorkersPerCu;
-    if (fp8) return bs <= 16 ? 8 : bs == 64 ? 3 : 4;
+    if (fp8) return bs <= 16 ? 8 : bs <= 32 ? 4 : 3;
     if (d <= 64) return bs <= 16 ? 8 : bs <= 32 ? 6 : 4;
     return bs * d > 16384 ? 4 : kWorkersPerCu;
 }

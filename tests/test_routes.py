@@ -141,3 +141,14 @@ def test_on_the_device(device):
         check_gqa(*row)
     for row in MLA:
         check_mla(*row)
+
+
+@pytest.mark.gpu
+def test_fp8_workers_by_block_size(device):
+    """Eight, four, three and three waves per CU (the default plan of long contexts)."""
+    import torch
+
+    cus = torch.cuda.get_device_properties(device).multi_processor_count
+    for bs, per_cu in ((16, 8), (32, 4), (64, 3), (128, 3)):
+        a = gqa(32, 8, 128, bs, 32, 1, 8192 // bs, kv_format=pa.KV_FP8_E4M3, k_scale=0x7000, v_scale=0x8000)
+        assert pa.plan(a) == cus * per_cu
