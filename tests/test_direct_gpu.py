@@ -1,6 +1,6 @@
 """The short-context decode (one workgroup per tile, no merge launch) at the
-edges of its shapes: fewer blocks than waves, one more, a last partial block,
-empty contexts, row tiles past the first, causal rows, the table widths on
+edges of its shapes: fewer blocks than waves, one more, several per wave, a last
+partial block, empty contexts, row tiles past the first, causal rows, the table widths on
 both sides of the rule that selects it, and its error reports."""
 
 from __future__ import annotations
@@ -80,6 +80,33 @@ def test_errors_are_reported(device):
     with pytest.raises(pa.PagedAttentionError) as e:
         pa.check_errors(device)
     assert e.value.rc == -6
+    pa.check_errors(device)
+
+
+# (heads, kv heads, dim, block, table width, lengths); several blocks per wave, so
+# a wave's K buffer is written block after block with the next one's loads in
+# flight, then holds its partial; waves of shorter sequences end early or idle
+@pytest.mark.parametrize("hq,hkv,dim,bs,width,lens", [
+    (8, 1, 128, 16, 24, [380, 17, 250]),                             # three blocks for a wave
+    (8, 2, 128, 16, 17, [272, 129]),
+    (32, 8, 128, 32, 24, [768, 500, 33, 97]),
+    (32, 8, 128, 128, 6, [768, 650, 257, 1] + [100 + 40 * i for i in range(12)]),  # 128 tiles, two blocks for a wave
+    (32, 8, 128, 16, 48, [768, 250, 641, 0] + [60 * i + 5 for i in range(12)]),
+    (8, 4, 256, 16, 16, [256, 241, 100, 129, 17, 1, 255, 64]),
+    (4, 2, 256, 128, 2, [206, 100, 130, 256]),                       # blocks larger than the registers, merged
+    (32, 8, 256, 128, 2, [206, 100] + [16 * i + 3 for i in range(14)]),
+])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_several_blocks_per_wave(hq, hkv, dim, bs, width, lens, dtype, device):
+    print(f"[case] {hq}/{hkv} d{dim} bs{bs} width {width} {lens} {dtype}", flush=True)
+    case = make_custom_case(batch=len(lens), num_heads=hq, kv_heads=hkv, head_dim=dim, block_size=bs,
+                            context_lens=lens, seed=1480 + dim + bs + width, dtype=dtype, max_blocks=width)
+    d = case.to(device)
+    out = torch.full(case.out_shape(), float("nan"), dtype=torch.float32, device=device)
+    args = pa.make_args(d.query, d.key_cache, d.value_cache, d.block_table, d.context_lens, out, case.scale)
+    assert pa.kernel_name(args) == "pa_direct_kernel"
+    pa.launch(args, device)
+    assert_close(out.cpu().numpy(), oracle_numpy(case), what=f"d{dim} bs{bs} width {width}")
     pa.check_errors(device)
 
 
