@@ -848,7 +848,7 @@ int simpler_launch_run(DeviceContextHandle h, RuntimeHandle runtime) {
     if (!set_device(c) || !r || r->magic != kRunMagic || r->state != 1) return -1;
     int rc;
     if (r->kind == kPagedAttention && r->execution == SIMPLER_HIP_EXEC_FUSED) {
-        // the merge kernel overwrites it; a batch of 0 launches nothing
+        // the last launch overwrites it; a batch of 0 launches nothing
         __atomic_store_n(c->err_host, 0u, __ATOMIC_RELEASE);
         rc = simpler_hip::pa_decode_with_mirror(&r->args, c->workspace, c->workspace_bytes, c->stream, c->err_host);
     } else {

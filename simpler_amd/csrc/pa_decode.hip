@@ -345,7 +345,7 @@ Plan make_plan(const SimplerHipPaDecodeArgs *a, const KernelPair &k) {  // k: th
 //   with two 12.2 / 9.4).
 // - To 128 tiles one block per wave or 48 KB (two 64 KB blocks 16.2 / 13.5).
 // - Every row tile of a kv head reads K and V again: with several of them up to
-//   64 KB per tile (0.93 at most, to 8192 tiles) or 48 MB in all (0.97 at most;
+//   64 KB per tile (0.93 at most, to 8192 tiles) or 48 MB in all (0.92 at most;
 //   128 x 8 kv heads, 64 rows of 64 dims, 1000 tokens in 32-token blocks, 1 GB,
 //   174 / 127; 15 x 8 of 380 tokens, 64 rows of 128 dims, 90 MB, 23.5 / 20.9).
 //   Above 64 dims, 768 KB over the row tiles of a kv head at most.
@@ -423,11 +423,12 @@ __global__ void mirror_kernel(const unsigned *flag, unsigned *mirror) {
 // It is shared out among workgroups (down to 8 units, a 128-byte line, each)
 // until a thread has one unit and reads kMergeAhead of its pieces at most,
 // as long as the grid stays within kMergeGrid workgroups: with more, every
-// workgroup's own set-up costs more than its shorter chain saves (128 x 128
-// MLA heads, 1024 tiles: 24.1 us with four per tile, 14.6 with one; 256
-// tiles: 14.6 against 19.9; one sequence of 16 heads and 32000 tokens, one
-// tile: 8 us in 128 workgroups, 321 in one). Small tiles of few pieces take
-// smaller workgroups.
+// workgroup's own set-up costs more than its shorter chain saves. us of the
+// merge alone, launched in a row: 128 sequences of 128 MLA heads, 1024 tiles,
+// 18.9 with one per tile and 30.9 with four; 32 of them, 256 tiles, 15.4 with
+// four, 16.2 with one, 17.8 with sixteen; one sequence of 16 heads and 32000
+// tokens, one tile, 7.2 in 128 workgroups and 444 in one. Small tiles of few
+// pieces take smaller workgroups.
 struct MergePlan {
     KernelFn fn;
     int units, groups, threads;
@@ -645,7 +646,12 @@ extern "C" int simpler_hip_pa_decode_append(const SimplerHipPaDecodeArgs *a, con
         // blocks measured slower (the verify shape: 155.2 against 140.2 us per
         // step), and MLA's register budget has no room for the new rows; with
         // one tile per worker the fused form is the faster one (cfg2: 113.3
-        // against 114.5).
+        // against 114.5). Ahead of the short-context kernel as well: both
+        // launches together against the fused work lists, on the device alone,
+        // 2 sequences of 153-512 tokens and one kv head 9.9 against 13.2 us, 16
+        // of 90-300 and 8 heads 9.2 against 12.3, 32 of 153-512 in 16-token
+        // blocks 13.3 against 18.3; 128 of 153-512, called in a row, 37.9
+        // against 42.8.
         const Kernels s = pick_kernel(a);
         if (s.k.main) {
             const Plan plan = make_plan(a, s.k);

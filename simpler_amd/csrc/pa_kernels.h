@@ -119,7 +119,7 @@ struct KernelParams {
     int32_t lanes;  // independent work lists; list u holds tiles [u, u+1) * (tiles per batch / lanes) of each batch
     float scale;
     int32_t causal;
-    unsigned *err_mirror;  // host-visible copy of *error_flag written by the merge kernel, or null
+    unsigned *err_mirror;  // host-visible copy of *error_flag written by the last launch, or null
     // Work units charged at the start of each work-list tile ahead of its
     // blocks (0: a slice's work is its block count). A slice that starts
     // further tiles pays for each one's set-up (query rows, first fill,
@@ -1518,8 +1518,8 @@ __global__ void __launch_bounds__(64 * MAXW) pa_decode_kernel(const KernelParams
 }
 
 // ---------------------------------------------------------------------------
-// Merge kernel: one workgroup per tile; log-sum-exp merge of the pieces
-// (pa_kernel.cce:1666-1773 CombineScale), and zeros for empty contexts.
+// Merge kernel: one or more workgroups per tile; log-sum-exp merge of the
+// pieces (pa_kernel.cce:1666-1773 CombineScale), and zeros for empty contexts.
 // ---------------------------------------------------------------------------
 
 constexpr int kMergeThreads = 512;  // largest merge workgroup
@@ -1623,7 +1623,10 @@ pa_merge_kernel(const KernelParams P) {
     auto piece_ml = [&](int k, int row) { return ml_base + (k * step + (k == 0 ? slot0 : 0)) * 32 + row; };
 
     const int r0 = unit0 / UPR, nr = (unit0 + units - 1) / UPR - r0 + 1;  // its rows
-    if (nr * np > kMergeTable) {  // contexts cut finer than the default plans cut
+    // More (row, piece) pairs than the table holds: a forced worker count, a very
+    // long context in small blocks (D = 16: 32000 tokens in 16-token blocks), or
+    // one long sequence in a large batch (plan_merge goes by the mean).
+    if (nr * np > kMergeTable) {
         for (int u = tid; u < units; u += MT) {
             const int row = (unit0 + u) / UPR;
             float M = -INFINITY;
