@@ -1524,7 +1524,7 @@ __global__ void __launch_bounds__(64 * MAXW) pa_decode_kernel(const KernelParams
 
 constexpr int kMergeThreads = 512;  // largest merge workgroup
 constexpr int kMergeAhead = 8;     // 16-byte units a thread reads before the weights are known
-constexpr int kMergeTable = 2048;  // (row, piece) weights a workgroup holds in LDS
+constexpr int kMergeTable = 1024;  // (row, piece) weights a workgroup holds in LDS
 
 // Combines x over a row of 16 lanes (DPP rotations); every lane gets the result.
 template <typename F>
@@ -1551,6 +1551,32 @@ __device__ __forceinline__ float row16_ordered_sum(const float c, const float l,
             c, l, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(L), 0x111, 0xf, 0xf, true)));  // row_shr:1
     return __int_as_float(
         __builtin_amdgcn_update_dpp(0, __float_as_int(L), 0x150 + N - 1, 0xf, 0xf, true));  // row_newbcast:N-1
+}
+
+// o += weight(x_k) v_k for k = k0, k0 + step, .. below np, in that order, N at a
+// time: load(k, x, v) reads one, and a batch's loads are all in flight together.
+template <int N, typename Load, typename Weight>
+__device__ __forceinline__ void add_pieces(std::integral_constant<int, N>, int k, const int step, const int np,
+                                           f32x4_t &o, Load load, Weight weight) {
+    for (; k + (N - 1) * step < np; k += N * step) {
+        float x[N];
+        f32x4_t v[N];
+#pragma unroll
+        for (int i = 0; i < N; ++i) load(k + i * step, x[i], v[i]);
+#pragma unroll
+        for (int i = 0; i < N; ++i) o += weight(x[i]) * v[i];
+    }
+    if (k < np) {  // the last batch, past its end: zeros
+        float x[N];
+        f32x4_t v[N];
+#pragma unroll
+        for (int i = 0; i < N; ++i) load(min(k + i * step, np - 1), x[i], v[i]);
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            const bool in = k + i * step < np;
+            o += (in ? weight(x[i]) : 0.f) * (in ? v[i] : (f32x4_t){0.f, 0.f, 0.f, 0.f});
+        }
+    }
 }
 
 // O = sum_w e^{m_w - M} O_w / L over a tile's pieces w. The merge is bound by
@@ -1623,29 +1649,85 @@ pa_merge_kernel(const KernelParams P) {
     auto piece_ml = [&](int k, int row) { return ml_base + (k * step + (k == 0 ? slot0 : 0)) * 32 + row; };
 
     const int r0 = unit0 / UPR, nr = (unit0 + units - 1) / UPR - r0 + 1;  // its rows
+    const int G = (UPT == 1 && np > PRE) ? MT / units : 1;  // piece groups
+    const int g = G > 1 ? tid / units : 0, u0 = tid - g * units;
+    __shared__ f32x4_t part[UPT == 1 ? kMergeThreads : 1];
+    // The groups' sums of a unit (UPT == 1) meet in group 0, which stores it.
+    auto finish = [&](f32x4_t o, int u) {
+        if (G > 1) {
+            part[tid] = o;
+            __syncthreads();
+            if (g == 0)
+                for (int i = 1; i < min(G, np); ++i) o += part[i * units + u0];
+        }
+        if (u < units && g == 0) OutStore<OutT>::store4(P.out, out_at(unit0 + u), o);
+    };
+
     // More (row, piece) pairs than the table holds: a forced worker count, a very
     // long context in small blocks (D = 16: 32000 tokens in 16-token blocks), or
-    // one long sequence in a large batch (plan_merge goes by the mean).
+    // one long sequence in a large batch (plan_merge goes by the mean). M and L
+    // of a row come from threads that take a piece of it each, the weights from
+    // each thread's own loads, kBatch pieces in flight. One thread per unit with
+    // four in flight, 64 sequences of 20-200 tokens with one of 100000, one kv
+    // head of 64 dims, 16-token blocks took 526 us per step; this way 47. (A
+    // table of 2048 pairs kept 200 sequences with one of 4000 at 25.6, 24.8 here.)
     if (nr * np > kMergeTable) {
-        for (int u = tid; u < units; u += MT) {
-            const int row = (unit0 + u) / UPR;
-            float M = -INFINITY;
-            for (int k = 0; k < np; ++k) M = fmaxf(M, *piece_ml(k, row));
-            float L = 0.f;
-            f32x4_t o = (f32x4_t){0.f, 0.f, 0.f, 0.f};
-#pragma unroll 4
-            for (int k = 0; k < np; ++k) {
-                const float c = __expf(*piece_ml(k, row) - M);
-                L += c * piece_ml(k, row)[16];
-                o += c * piece_unit(k, unit0 + u);
+        constexpr int kBatch = 8 / UPT;
+        constexpr int kBatchMl = 4;
+        __shared__ float sm[kMergeThreads / 64][16], sl[kMergeThreads / 64][16], row_m[16], row_inv[16];
+        float M = -INFINITY, L = 0.f;  // of row tid % 16 over the pieces tid / 16, + MT / 16, ..
+        const int r = min(tid & 15, nr - 1), per = MT >> 4;
+        for (int k = tid >> 4; k < np; k += kBatchMl * per) {
+            float m[kBatchMl], l[kBatchMl];
+#pragma unroll
+            for (int i = 0; i < kBatchMl; ++i) {
+                const float *ml = piece_ml(min(k + i * per, np - 1), r0 + r);
+                m[i] = ml[0];
+                l[i] = k + i * per < np ? ml[16] : 0.f;
             }
-            OutStore<OutT>::store4(P.out, out_at(unit0 + u), L > 0.f ? o / L : (f32x4_t){0.f, 0.f, 0.f, 0.f});
+            float Mn = M;
+#pragma unroll
+            for (int i = 0; i < kBatchMl; ++i) Mn = fmaxf(Mn, m[i]);
+            L *= __expf(M - Mn);
+#pragma unroll
+            for (int i = 0; i < kBatchMl; ++i) L += __expf(m[i] - Mn) * l[i];
+            M = Mn;
+        }
+        auto join = [](float &M0, float &L0, const float M1, const float L1) {  // (-inf, 0): no piece
+            const float Mn = fmaxf(M0, M1);
+            L0 = (L0 > 0.f ? L0 * __expf(M0 - Mn) : 0.f) + (L1 > 0.f ? L1 * __expf(M1 - Mn) : 0.f);
+            M0 = Mn;
+        };
+        join(M, L, __shfl_xor(M, 16, 64), __shfl_xor(L, 16, 64));
+        join(M, L, __shfl_xor(M, 32, 64), __shfl_xor(L, 32, 64));
+        if ((tid & 63) < 16) {
+            sm[tid >> 6][tid & 15] = M;
+            sl[tid >> 6][tid & 15] = L;
+        }
+        __syncthreads();
+        if (tid < nr) {
+            for (int w = 1; w < MT >> 6; ++w) join(M, L, sm[w][tid], sl[w][tid]);
+            row_m[tid] = M;
+            row_inv[tid] = L > 0.f ? 1.f / L : 0.f;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int n = 0; n < UPT; ++n) {
+            const int u = u0 + n * MT;
+            f32x4_t o = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+            if (u < units && g < G) {
+                const int row = (unit0 + u) / UPR;
+                const float Mr = row_m[row - r0], inv = row_inv[row - r0];
+                add_pieces(std::integral_constant<int, kBatch>{}, g, G, np, o, [&](int k, float &w, f32x4_t &v) {
+                    v = piece_unit(k, unit0 + u);
+                    w = *piece_ml(k, row);
+                }, [&](float m) { return __expf(m - Mr) * inv; });
+            }
+            finish(o, u);
         }
         return;
     }
 
-    const int G = (UPT == 1 && np > PRE) ? MT / units : 1;  // piece groups
-    const int g = G > 1 ? tid / units : 0, u0 = tid - g * units;
     f32x4_t pre[UPT][PRE];
 #pragma unroll
     for (int n = 0; n < UPT; ++n) {
@@ -1661,7 +1743,6 @@ pa_merge_kernel(const KernelParams P) {
     // the short-context kernel does: both give the same bits for the same
     // pieces.
     __shared__ float wgt[kMergeTable], lsum[kMergeTable];  // [row][piece]: m, then its weight; l
-    __shared__ f32x4_t part[UPT == 1 ? kMergeThreads : 1];
     for (int e = tid; e < nr * np; e += MT) {  // all (m, l) loads in flight at once
         const int r = e / np;
         const float *ml = piece_ml(e - r * np, r0 + r);
@@ -1716,19 +1797,19 @@ pa_merge_kernel(const KernelParams P) {
 #pragma unroll
             for (int i = 0; i < PRE; ++i)
                 if (g + i * G < np) o += w[g + i * G] * pre[n][i];
+            if constexpr (UPT == 4) {
 #pragma unroll 4
-            for (int k = g + PRE * G; k < np; k += G) o += w[k] * piece_unit(k, unit0 + u);
+                for (int k = PRE; k < np; ++k) o += w[k] * piece_unit(k, unit0 + u);
+            } else {
+                add_pieces(std::integral_constant<int, PRE>{}, g + PRE * G, G, np, o, [&](int k, float &c, f32x4_t &v) {
+                    v = piece_unit(k, unit0 + u);
+                    c = w[k];
+                }, [](float c) { return c; });
+            }
         }
-        if (G > 1) {  // (UPT == 1)
-            part[tid] = o;
-            __syncthreads();
-            if (g == 0)
-                for (int i = 1; i < min(G, np); ++i) o += part[i * units + u0];
-        }
-        if (u < units && g == 0) OutStore<OutT>::store4(P.out, out_at(unit0 + u), o);
+        finish(o, u);
     }
 }
-
 
 // ---------------------------------------------------------------------------
 // MLA decode: one latent KV head shared by every query head (Hkv = 1 in the

@@ -1,7 +1,7 @@
 """The split merge at the edges of its launch shapes: tiles of one row up to a
 full 16, every output width, and contexts cut into few pieces (one workgroup
 per tile), many (several workgroups and groups of threads per tile) and more
-than its LDS table of weights holds (2048 per workgroup)."""
+than its LDS table of weights holds (1024 per workgroup)."""
 
 from __future__ import annotations
 
@@ -26,6 +26,11 @@ pytestmark = pytest.mark.gpu
     (16, 256, [130, 7, 1], 3),     # more units than threads, few pieces
     (16, 32, [2300], 5000),        # above the LDS table: 16 rows x 2300 pieces
     (20, 64, [50, 33], 40),        # a second row tile of 4 rows
+    # above the LDS table in a batch whose mean is short: one workgroup per tile
+    (16, 64, [300] + [1] * 69, 369),
+    (16, 16, [300] + [1] * 69, 369),   # several groups of threads
+    (5, 128, [2, 500, 0, 1] + [1] * 60, 570),
+    (16, 256, [200] + [1] * 599, 799),  # two units per thread
 ])
 def test_pieces_and_rows(group, dim, blocks, workers, device):
     print(f"[case] group={group} dim={dim} blocks={blocks} workers={workers}", flush=True)
@@ -39,7 +44,11 @@ def test_pieces_and_rows(group, dim, blocks, workers, device):
     pa.check_errors(device)
 
 
-@pytest.mark.parametrize("heads,lens,workers", [(16, [3000], 90), (33, [700, 0, 64], 12), (128, [500] * 3, 6)])
+@pytest.mark.parametrize("heads,lens,workers", [
+    (16, [3000], 90), (33, [700, 0, 64], 12), (128, [500] * 3, 6),
+    (16, [9000] + [32] * 40, 800),    # above the LDS table
+    (128, [4800] + [32] * 66, 760),   # the same with four units per thread
+])
 def test_mla_pieces(heads, lens, workers, device):
     print(f"[case] mla heads={heads} lens={lens} workers={workers}", flush=True)
     case = make_custom_case(batch=len(lens), num_heads=heads, kv_heads=1, head_dim=576, head_dim_v=512, block_size=32,
