@@ -216,12 +216,12 @@ int wave_slots(KernelFn fn, int threads, int want_per_cu, size_t lds = 0) {
 //   3 / 4 tiles, 35.7 / 40.0 against 49.9 / 52.6 (at 64 and 128 tokens one
 //   workgroup is best); fp8, 2 tiles, 16 / 32 / 64 tokens 42.7 / 35.3 / 34.1
 //   against 75.1 / 51.4 / 41.0.
-// A plan made without a device (which can launch nothing) reports nominal
+// A plan made without a device (which can launch nothing) reports `nominal`
 // counts that do not depend on the block size.
-int workers_per_cu(const SimplerHipPaDecodeArgs *a, const KernelPair &k, const Plan &p, bool pair) {
+int workers_per_cu(const SimplerHipPaDecodeArgs *a, const KernelPair &k, const Plan &p, bool pair, bool nominal) {
     if (pair) return kWorkersThreePerCu;
     const int bs = a->block_size, d = a->head_dim_k, tiles = p.tiles_per_worker;
-    const bool fp8 = a->kv_format == SIMPLER_HIP_KV_FP8_E4M3, nominal = current_device() < 0;
+    const bool fp8 = a->kv_format == SIMPLER_HIP_KV_FP8_E4M3;
     if (tiles > 1) {
         if (nominal) return kWorkersPerCu;
         const int waves = (d <= 64 || fp8) ? (bs <= 16 ? 12 : bs <= 32 ? 9 : bs <= 64 ? 6 : 4)
@@ -282,7 +282,7 @@ Plan make_plan(const SimplerHipPaDecodeArgs *a, const KernelPair &k) {  // k: th
         if (!pair && k.klds && p.tiles_per_worker > 1) p.lds = (size_t)p.tiles_per_worker * a->block_size * 256;
         p.groups = 1;
         p.row_groups = (p.row_tiles + p.tiles_per_worker - 1) / p.tiles_per_worker;
-        const int per_cu = workers_per_cu(a, k, p, pair);
+        const int per_cu = workers_per_cu(a, k, p, pair, current_device() < 0);
         p.workers = a->num_workers > 0 ? a->num_workers : wave_slots(p.main, p.threads, per_cu, p.lds);
         // Work lists (the tiles of a batch shared out among them, rotating with
         // the batch). 16-bit caches: one list per tile of a batch when the
@@ -344,6 +344,12 @@ Plan make_plan(const SimplerHipPaDecodeArgs *a, const KernelPair &k) {  // k: th
 //   most; 9.8 / 9.6 at 384), with 256 dims one block per wave (1.005 at most;
 //   with two 12.2 / 9.4).
 // - To 128 tiles one block per wave or 48 KB (two 64 KB blocks 16.2 / 13.5).
+// - A sequence as long as the table among short ones is one chain here, and cut
+//   among all workers by the lists: to 511 tiles six blocks per wave to 32
+//   tokens, four of 64, three of 128, from 512 tiles ten, ten, six and three.
+//   With one such sequence and 10 tokens in the others 0.96 at most (512 tiles
+//   of 16 dims, 64-token blocks: 6 blocks 0.9, 8 15.7 / 14.1, 32 51.6 / 15.0;
+//   2048 of 64 dims, 32-token blocks: 8 0.73, 16 23.3 / 18.9, 32 42.3 / 19.4).
 // - Every row tile of a kv head reads K and V again: with several of them up to
 //   64 KB per tile (0.93 at most, to 8192 tiles) or 48 MB in all (0.92 at most;
 //   128 x 8 kv heads, 64 rows of 64 dims, 1000 tokens in 32-token blocks, 1 GB,
@@ -361,9 +367,10 @@ int direct_waves(const SimplerHipPaDecodeArgs *a, const Kernels &s, const Plan &
     if (!narrow && p.row_tiles > 1 && tile * p.row_tiles > 768 * KB) return 0;
     Plan one = p;
     one.tiles_per_worker = 1;
-    const int64_t want = (int64_t)cu_count() * std::max(kWorkersPerSimdCu, workers_per_cu(a, s.k, one, false));
+    const int64_t want = (int64_t)cu_count() * std::max(kWorkersPerSimdCu, workers_per_cu(a, s.k, one, false, false));
     const int64_t waves = std::min<int64_t>({(want + tiles - 1) / tiles, s.direct.max_waves, blocks});
     const int64_t per_wave = (blocks + waves - 1) / waves;
+    if (per_wave > (bs > 64 ? 3 : bs > 32 ? (tiles < 512 ? 4 : 6) : (tiles < 512 ? 6 : 10))) return 0;
     if (tiles < 128 && per_wave > 1 && per_wave * block > 48 * KB) return 0;
     if (tiles < 32 && per_wave > 1 && d > 128) return 0;
     const int64_t most = narrow    ? (tiles < 32 ? 192 : 256)
@@ -379,24 +386,27 @@ int direct_waves(const SimplerHipPaDecodeArgs *a, const Kernels &s, const Plan &
 // host knows the table's width and not the lengths: with few workgroups a tile
 // cut into blocks ends earlier. us per step against the work lists, 16 / 64 /
 // 128 rows, 64-token blocks:
-// - to 128 tokens always: one sequence 10.6 / 15.5 / 21.1 against 13.5 / 18.1 /
+// - to 128 tokens any: one sequence 10.6 / 15.5 / 21.1 against 13.5 / 18.1 /
 //   23.0, 128 of them 11.7 / 17.6 / 23.9 against 19.8 / 27.9 / 35.6;
 // - to 256 from 32 workgroups: 32 of 128-256 tokens 14.5 / 20.3 / 28.9 against
 //   15.3 / 26.3 / 31.6 (8 of them 14.5 / 20.0 / 28.1 against 14.0 / 20.0 / 26.5);
 // - to 512 from 128 workgroups: 128 of 64-512 tokens 23.3 / 31.0 / 43.9 against
 //   26.7 / 38.8 / 52.4 (64 of 256-512 22.9 / 30.3 / 43.1 against 20.5 / 31.5 /
 //   41.7; 300 of 256-1024 73 / 87 / 120 against 69 / 88 / 121).
-// 32-token blocks are twice the steps: a quarter less where the workgroups are
-// fewest, below 8 (one sequence of 128 tokens, 96 rows 20.4 against 19.2; of 96
-// 0.95 of the lists' time at most) and from 32 to 63 (32 of 51-256 tokens, 16
-// rows 16.7 against 15.8; 0.93 at most to 192, and to 256 from 64 workgroups).
+// These are with lengths near each other; one sequence as long as the table
+// among sequences of 10 tokens is a chain of blocks here, hence 384 tokens from
+// 128 workgroups (128 rows 42.1 against 38.0 at 512) and 192 below 64 (128 rows
+// 27.8 against 26.6 at 256). 32-token blocks are twice the steps: 256 tokens from
+// 128 workgroups (128 of 128 rows 52.0 against 40.2 at 512), 192 from 64 (64 of
+// 16 rows 15.9 against 15.3 at 256), 160 from 32, else 96 (one sequence of 128
+// tokens, 96 rows, 20.4 against 19.2). 0.98 of the lists' time at most, 1.00 for
+// 64 rows with 32-token blocks.
 bool mla_whole_tiles(const SimplerHipPaDecodeArgs *a, const Kernels &s, const Plan &p) {
     if (!s.k.mla || a->num_workers > 0) return false;
     const int64_t groups = (int64_t)a->batch * a->num_kv_heads * p.groups;
     const int64_t tokens = (int64_t)a->max_blocks_per_seq * a->block_size;
-    int64_t most = groups >= 128 ? 512 : groups >= 32 ? 256 : 128;
-    if (a->block_size == 32 && (groups < 8 || (groups >= 32 && groups < 64))) most -= most / 4;
-    return tokens <= most;
+    if (a->block_size == 32) return tokens <= (groups >= 128 ? 256 : groups >= 64 ? 192 : groups >= 32 ? 160 : 96);
+    return tokens <= (groups >= 128 ? 384 : groups >= 64 ? 256 : groups >= 32 ? 192 : 128);
 }
 
 // How a plain decode runs: one workgroup of `waves` waves per tile

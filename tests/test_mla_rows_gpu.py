@@ -44,10 +44,17 @@ def test_few_rows(bs, heads, q_len, lens, workers, scale, device):
     (65, 1, 2, 32, 5, 4, 128),       # two row groups, the second partly filled
     (16, 1, 1, 64, 2, 3, 192),       # too long for two workgroups: work lists
     (33, 1, 1, 64, 32, 4, 256),      # 32 workgroups
-    (4, 2, 4, 32, 16, 6, 192),       # two kv heads
-    (4, 2, 4, 32, 16, 8, 256),       # too long for 32 workgroups with 32-token blocks: work lists
+    (4, 2, 4, 32, 16, 8, 256),       # two kv heads
     (128, 1, 2, 64, 64, 8, 512),     # 128 workgroups
     (16, 1, 1, 64, 129, 8, 512),
+    # the longest whole tiles of each range (those above are just past it)
+    (65, 1, 2, 32, 5, 3, 96),
+    (33, 1, 1, 64, 32, 3, 192),
+    (16, 1, 1, 64, 64, 4, 256),
+    (4, 2, 4, 32, 16, 5, 160),
+    (128, 1, 2, 64, 64, 6, 384),
+    (16, 1, 1, 64, 129, 6, 384),
+    (16, 1, 1, 32, 128, 8, 256),
 ])
 def test_whole_tiles(heads, kv_heads, q_len, bs, batch, width, longest, device):
     """Against the oracle and the work lists (a forced worker count)."""

@@ -53,6 +53,17 @@ GQA = [
     (32, 8, 256, 64, 16, 1, 7, False),
     (32, 8, 256, 128, 16, 1, 2, True),  # blocks larger than the registers
     (32, 8, 256, 128, 16, 1, 3, False),
+    # the blocks of one wave
+    (32, 8, 16, 16, 16, 1, 96, True),   # six of 16 waves
+    (32, 8, 16, 16, 16, 1, 97, False),
+    (4, 1, 16, 64, 1, 1, 32, True),     # four of 8
+    (4, 1, 16, 64, 1, 1, 33, False),
+    (4, 1, 16, 128, 1, 1, 12, True),    # three of 4
+    (4, 1, 16, 128, 1, 1, 13, False),
+    (32, 8, 64, 32, 64, 1, 30, True),   # 512 tiles: ten of 3
+    (32, 8, 64, 32, 64, 1, 31, False),
+    (32, 8, 128, 64, 256, 1, 6, True),  # 2048 tiles: six of one
+    (32, 8, 128, 64, 256, 1, 7, False),
     # several row tiles: 64 KB per tile or 48 MB over all of them
     (128, 8, 64, 32, 32, 4, 8, True),
     (128, 8, 64, 32, 32, 4, 9, False),
@@ -85,22 +96,24 @@ def check_gqa(hq, hkv, d, bs, batch, q_len, width, short, **kw):
 MLA = [
     (16, 1, 1, 1, 64, 2, True),
     (16, 1, 2, 1, 64, 3, False),
-    (65, 1, 5, 2, 32, 4, True),
-    (33, 1, 32, 1, 64, 4, True),
-    (33, 1, 31, 1, 64, 4, False),
-    (4, 2, 16, 4, 32, 4, True),
-    (128, 1, 64, 2, 64, 8, True),
-    (128, 1, 63, 2, 64, 8, False),
-    (16, 1, 129, 1, 64, 8, True),
-    (16, 1, 129, 1, 64, 9, False),
-    # 32-token blocks with the fewest workgroups of each range
-    (96, 1, 7, 1, 32, 3, True),
+    (33, 1, 32, 1, 64, 3, True),     # 192 tokens from 32 workgroups
+    (33, 1, 32, 1, 64, 4, False),
+    (33, 1, 31, 1, 64, 3, False),
+    (16, 1, 64, 1, 64, 4, True),     # 256 from 64
+    (16, 1, 64, 1, 64, 5, False),
+    (128, 1, 64, 2, 64, 6, True),    # 384 from 128
+    (128, 1, 63, 2, 64, 6, False),
+    (16, 1, 129, 1, 64, 6, True),
+    (16, 1, 129, 1, 64, 7, False),
+    # 32-token blocks
+    (65, 1, 5, 2, 32, 3, True),
     (96, 1, 7, 1, 32, 4, False),
-    (96, 1, 8, 1, 32, 4, True),
-    (16, 1, 32, 1, 32, 6, True),
-    (16, 1, 32, 1, 32, 7, False),
-    (16, 1, 63, 1, 32, 7, False),
-    (16, 1, 64, 1, 32, 8, True),
+    (4, 2, 16, 4, 32, 5, True),
+    (16, 1, 32, 1, 32, 6, False),
+    (16, 1, 64, 1, 32, 6, True),
+    (16, 1, 127, 1, 32, 7, False),
+    (16, 1, 128, 1, 32, 8, True),
+    (16, 1, 128, 1, 32, 9, False),
 ]
 
 
